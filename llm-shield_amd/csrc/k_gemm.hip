@@ -19,12 +19,12 @@
 // bit-identical to running its branches one at a time.  Tile shapes may
 // therefore be chosen by M without changing a single bit.
 //
-// Pipeline.  K advances 64 (two quant blocks) per stage.  Weights stream from
-// HBM as raw quant bytes into registers two stages ahead, are decoded to fp16
-// integers into a double-buffered LDS tile one stage ahead ("dequant in LDS":
-// each decoded weight feeds every row of the tile), and the activation
-// fragments are loaded straight from global memory (L2-resident) into the
-// MFMA operand registers one stage ahead.  One barrier per stage.
+// Pipeline.  K advances 64 (two quant blocks) per stage.  The waves of a
+// workgroup sit side by side along N; each streams its own weight tiles from
+// HBM as raw quant bytes into registers two stages ahead and decodes them
+// there (a tile slot is the lane's B fragment), while the stage's activation
+// tile goes to LDS once per workgroup, double buffered, and serves every wave.
+// One barrier per stage.
 //
 // Outputs.  Store-mode results (and K-split partials) are written with
 // nontemporal stores: their consumer runs on whichever XCD its workgroup lands
@@ -33,12 +33,10 @@
 // to back took 1-6 % less time (QKV 25.4 -> 24.8 us, O 18.7 -> 17.8, down
 // 34.9 -> 34.3); in the model, between other kernels, under 0.5 %.
 //
-// Tiles.  4 waves.  This dequant-in-LDS kernel serves segment lists the
-// B-direct kernel below cannot split (64 x 64 tiles at small M, 128 x 128 at
-// large M); the B-direct kernel takes everything else.  Workgroup ids are remapped so each XCD (ids round-robin over 8) works on a
-// contiguous run of a grouped tile order: neighbouring tiles on one XCD share
-// weight and activation tiles in its L2.  LDS rows are padded to 72 halves
-// (144 B) so 16-byte fragment reads of 8 lanes hit distinct banks.
+// Tiles.  16 TM x 16 TN per wave, four to sixteen waves per workgroup, chosen
+// by the shape (launch_mode).  Workgroup ids are remapped so each XCD (ids
+// round-robin over 8) works on a contiguous run of a grouped tile order:
+// neighbouring tiles on one XCD share weight and activation tiles in its L2.
 #include "jev_dev.h"
 
 #include <type_traits>
@@ -47,467 +45,85 @@ namespace jev {
 
 namespace {
 
-constexpr int BK = 64;           // K per stage (two quant blocks)
-constexpr int LROW = BK + 8;     // padded LDS row, halves
-
-struct alignas(16) u32x4 {
-    uint32_t x, y, z, w;
-};
-
-
 // One loader chunk: a lane slot of a weight tile -- the quants of one row
 // at k = 8g .. 8g + 7 of both blocks of the stage -- and that row's scales.
 struct BChunk {
-    uint4 q;       // bytes (Q8_0, Q5_1's byte copy): 16; nibbles (Q4_0, Q5_1's fields): 8 in .x, .y
+    uint4 q;       // bytes (Q8_0, Q5_1's byte copy): 16; nibbles (Q4_0): 8 in .x, .y
     uint32_t d, m; // two fp16 each (block 0 low half)
-    uint32_t qh;   // Q5_1 from its 5-bit fields: the lane's fifth bits (block 0 low byte)
 };
-
-// Segment and local row of tile column rr (epilogue).
-template <int MODE, int BN>
-__device__ __forceinline__ void map_row(const GemmArgs &a, int tile_n, int rr, int &seg, int &row)
-{
-    if (MODE == kGemmSwiGlu) {
-        int sub = rr >> 4;
-        seg = sub & 1;
-        row = tile_n * (BN / 2) + (sub >> 1) * 16 + (rr & 15);
-    } else {
-        int n0 = tile_n * BN;
-        int s = 0, start = 0;
-        while (s + 1 < a.nseg && n0 >= start + a.seg[s].rows) {
-            start += a.seg[s].rows;
-            s++;
-        }
-        seg = s;
-        row = n0 - start + rr;
-    }
-}
 
 // Loads are unconditional with clamped addresses: a row past the weight's end
 // or a block past K only feeds outputs that are never stored, and keeping the
 // loop free of divergent loads lets the compiler count outstanding loads
 // exactly instead of draining the queue every stage.
 
-// Quants as these kernels read them.  BQ (byte quants): whole bytes, 1 KiB
-// per tile -- Q8_0's (QWeight::qs, stored biased as q + 128) or Q5_1's byte
-// copy (QWeight::qb, q itself).  Otherwise 512 B of nibbles per tile (QWeight::qs:
-// Q4_0, or Q5_1's low four bits with the fifth bits in QWeight::qh).  Q8_0
-// is always bytes, Q4_0 always nibbles; Q5_1 is bytes wherever the kernel's
-// registers allow the 16-byte chunk (all but the 64 x 256 tile): one byte
-// permute and one packed subtraction per two weights instead of the nibble
-// and fifth-bit assembly.  The decoded integers are the same either way.
-template <int TYPE, bool BQ>
+// Quants as these kernels read them: whole bytes, 1 KiB per tile -- Q8_0's
+// (QWeight::qs, stored biased as q + 128) or Q5_1's byte copy (QWeight::qb, q
+// itself: one byte permute and one packed subtraction per two weights instead
+// of the nibble and fifth-bit assembly) -- or Q4_0's nibbles, 512 B per tile.
+template <int TYPE>
+constexpr bool kByteQuants = TYPE != kQ4_0;
+
+template <int TYPE>
 __device__ __forceinline__ rsrc_t quant_rsrc(const QWeight &w, uint32_t tiles)
 {
-    return make_rsrc(TYPE == kQ5_1 && BQ ? w.qb : w.qs, tiles * (BQ ? 1024u : 512u));
+    return make_rsrc(TYPE == kQ5_1 ? w.qb : w.qs, tiles * (kByteQuants<TYPE> ? 1024u : 512u));
 }
 
 // Four quants of a block as two fp16 pairs of exact integers: a byte b placed
 // under the exponent byte is 1024 + b; the bias subtracts 1024 and, for Q8_0's
 // biased bytes or Q4_0's offset 8, that too.
-template <int TYPE, bool BQ>
+template <int TYPE>
 __device__ __forceinline__ void decode4(const BChunk &c, int bb, int half, uint32_t &pa, uint32_t &pb)
 {
-    if (BQ) {
+    if (kByteQuants<TYPE>) {
         const uint32_t w = bb ? (half ? c.q.w : c.q.z) : (half ? c.q.y : c.q.x);
         bytes_to_f16(w, TYPE == kQ8_0 ? (_Float16)1152.0f : (_Float16)1024.0f, pa, pb);
     } else {
         // byte i = element i (low nibble) | element i + 4 (high nibble)
         const uint32_t w = bb ? c.q.y : c.q.x;
-        uint32_t n = half ? (w >> 4) & 0x0f0f0f0fu : w & 0x0f0f0f0fu;
-        _Float16 bias = (_Float16)1032.0f;
-        if (TYPE == kQ5_1) {
-            // fifth bits: spread 4 bits to bit 4 of each byte
-            const uint32_t hb = (c.qh >> (8 * bb)) & 0xffu;
-            n |= ((((half ? hb >> 4 : hb & 15u)) * 0x00204081u) & 0x01010101u) << 4;
-            bias = (_Float16)1024.0f;
-        }
-        bytes_to_f16(n, bias, pa, pb);
+        const uint32_t n = half ? (w >> 4) & 0x0f0f0f0fu : w & 0x0f0f0f0fu;
+        bytes_to_f16(n, (_Float16)1032.0f, pa, pb);
     }
 }
 
 // B fragment of block bb of a loaded chunk: 8 fp16 integers for the lane's
 // row at k = 8g .. 8g + 7.
-template <int TYPE, bool BQ>
+template <int TYPE>
 __device__ __forceinline__ half8_t decode_b_frag(const BChunk &c, int bb)
 {
     uint32_t o0, o1, o2, o3;
-    decode4<TYPE, BQ>(c, bb, 0, o0, o1);
-    decode4<TYPE, BQ>(c, bb, 1, o2, o3);
+    decode4<TYPE>(c, bb, 0, o0, o1);
+    decode4<TYPE>(c, bb, 1, o2, o3);
     return __builtin_bit_cast(half8_t, make_uint4(o0, o1, o2, o3));
 }
 
-// Decoded quants of one chunk as fp16 integers: block 0 to dst[0..8),
-// block 1 to dst[32..40) (the LDS row of the chunk's weight row).
-template <int TYPE, bool BQ>
-__device__ __forceinline__ void store_chunk(const BChunk &c, uint16_t *dst)
-{
-#pragma unroll
-    for (int bb = 0; bb < 2; bb++) {
-        uint32_t o0, o1, o2, o3;
-        decode4<TYPE, BQ>(c, bb, 0, o0, o1);
-        decode4<TYPE, BQ>(c, bb, 1, o2, o3);
-        *(u32x4 *)(dst + 32 * bb) = u32x4{o0, o1, o2, o3};
-    }
-}
-
-// A fragments of one stage: [mi][kb2] hi and lo.
-template <int TM>
-struct AFrag {
-    half8_t hi[TM][2], lo[TM][2];
-    floatx4 s[TM][2]; // Q5_1 block sums of the lane's 4 C rows
-};
-
 } // namespace
 
-// KS: quant blocks whose partials are in flight together (1 or 2); OCC:
-// waves per SIMD the register budget is cut for.
-template <int TYPE, int MODE, int WM, int WN, int TM, int TN, int PD, int KS, int OCC>
-__global__ __launch_bounds__(256, OCC) void gemm_q_kernel(GemmArgs a, int mt, int nt, int gm)
-{
-    constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
-    constexpr int CHUNKS = BN * 4; // 64 lane slots per 16-row weight tile
-    constexpr int CPT = (CHUNKS + 255) / 256;
-    constexpr int NG = TN < 4 ? TN : 4; // N tiles per partial group
-    // One spare chunk / scale slot past each tile: loaders with nothing to
-    // store write there, so no store (and no wait on its load) is conditional.
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[2][BN * LROW + 40];
-    __shared__ float Ds[2][BN * 2 + 2];
-    __shared__ float Ms[2][TYPE == kQ5_1 ? BN * 2 + 2 : 1];
-
-    // ---- tile of this workgroup: contiguous per-XCD runs of a grouped order
-    const int total = gridDim.x;
-    const int per_xcd = total >> 3;
-    const int L = blockIdx.x;
-    int Lp = (L & 7) * per_xcd + (L >> 3);
-    // K split z (partials of store-mode GEMMs): whole runs of the tile order
-    const int tiles8 = total / a.ksplit;
-    const int z = Lp / tiles8;
-    Lp -= z * tiles8;
-    const int group = gm * nt;
-    const int first_m = (Lp / group) * gm;
-    const int gsz = min(mt - first_m, gm);
-    if (gsz <= 0) return;
-    const int tile_m = first_m + (Lp % group) % gsz;
-    const int tile_n = (Lp % group) / gsz;
-    if (tile_m >= mt || tile_n >= nt) return;
-
-    // wave-uniform in a scalar register (a vector value can turn the loads'
-    // scalar offsets into per-lane loops)
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WN, wn = wave % WN;
-    const int M = a.M, K = a.K, nblk = K >> 5;
-    // this split's K blocks: [kb_begin, kb_begin + nb)
-    const int nb_per = gemm_split_blocks(nblk, a.ksplit);
-    const int kb_begin = z * nb_per;
-    const int nb = min(nblk - kb_begin, nb_per);
-    const int nstage = (nb + 1) >> 1;
-    const int m0 = tile_m * BM;
-
-    // ---- loader role (B): chunk c = tid + 256 j is lane slot c % 64 of the
-    // tile row c / 64 of the workgroup's BN weight rows -- one tile per wave,
-    // so its weight (segment) is uniform.  Every load is a buffer load: a
-    // scalar resource, a per-lane offset fixed for the loop and a scalar
-    // per-stage offset; no per-stage vector address arithmetic.
-    rsrc_t rq[CPT], rd[CPT];
-    int btile0[CPT]; // first tile of the chunk's row group (uniform)
-    int b_lds[CPT], b_ds[CPT];
-    const int slot = tid & 63, sg = slot >> 4, sr = slot & 15;
-    constexpr bool BQ = TYPE != kQ4_0; // byte quants (see quant_rsrc)
-    const uint32_t vq = (uint32_t)slot * (BQ ? 16 : 8), vd = 4 * sr;
-    const int kp_begin = kb_begin >> 1; // kb_begin is even
-#pragma unroll
-    for (int j = 0; j < CPT; j++) {
-        const int t = wave + 4 * j; // tile row within the workgroup
-        const bool own = 16 * t < BN; // waves past the tile load a duplicate and store it in the spare slot
-        int seg, rgw;
-        if (MODE == kGemmSwiGlu) {
-            // 16-row groups alternate gate (segment 0) and up (segment 1)
-            seg = t & 1;
-            rgw = tile_n * (BN / 32) + (t >> 1);
-        } else {
-            int s0 = 0, start = 0, n0 = tile_n * BN;
-            while (s0 + 1 < a.nseg && n0 >= start + a.seg[s0].rows) {
-                start += a.seg[s0].rows;
-                s0++;
-            }
-            seg = s0;
-            rgw = (n0 - start) / 16 + t; // segments but the last are whole tiles
-        }
-        seg = __builtin_amdgcn_readfirstlane(seg);
-        const QWeight &w = a.seg[seg];
-        const int KP = tile_kpairs(w.cols), RG = tile_rows(w.rows);
-        const uint32_t tiles = (uint32_t)RG * KP;
-        rq[j] = quant_rsrc<TYPE, BQ>(w, tiles);
-        rd[j] = make_rsrc(w.d, tiles * tile_d_bytes(TYPE));
-        // row groups past the weight feed unstored columns
-        btile0[j] = __builtin_amdgcn_readfirstlane(min(rgw, RG - 1) * KP + kp_begin);
-        b_lds[j] = own ? (16 * t + sr) * LROW + 8 * sg : BN * LROW;
-        // lanes of the first k group store the row's two scales, the rest the spare slot
-        b_ds[j] = own && sg == 0 ? (16 * t + sr) * 2 : BN * 2;
-    }
-    // A stage past the end reloads the last one.  An odd block count leaves
-    // the last stage's second block to the tile padding (zero quants and
-    // scales) or to the next split's first block; either way it only feeds
-    // the skipped second half.
-    auto load_b = [&](int st, BChunk (&br)[CPT]) {
-        st = min(st, nstage - 1);
-#pragma unroll
-        for (int j = 0; j < CPT; j++) {
-            const int tile = btile0[j] + st;
-            if (BQ) {
-                br[j].q = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rq[j], vq, tile * 1024, 0));
-            } else {
-                uint2 v = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rq[j], vq, tile * 512, 0));
-                br[j].q = make_uint4(v.x, v.y, 0u, 0u);
-            }
-            if (TYPE == kQ5_1) {
-                // the row's scales and mins in one load
-                const uint2 dm = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rd[j], 2 * vd, tile * 128, 0));
-                br[j].d = dm.x;
-                br[j].m = dm.y;
-            } else {
-                br[j].d = __builtin_amdgcn_raw_buffer_load_b32(rd[j], vd, tile * 64, 0);
-            }
-        }
-    };
-    auto store_b = [&](int buf, const BChunk (&br)[CPT]) {
-#pragma unroll
-        for (int j = 0; j < CPT; j++) {
-            store_chunk<TYPE, BQ>(br[j], &Bs[buf][b_lds[j]]);
-            Ds[buf][b_ds[j]] = h2f((uint16_t)br[j].d);
-            Ds[buf][b_ds[j] + 1] = h2f((uint16_t)(br[j].d >> 16));
-            if (TYPE == kQ5_1) {
-                Ms[buf][b_ds[j]] = h2f((uint16_t)br[j].m);
-                Ms[buf][b_ds[j] + 1] = h2f((uint16_t)(br[j].m >> 16));
-            }
-        }
-    };
-
-    // ---- A fragments straight from global memory: each is one contiguous
-    // 1 KiB operand tile (xt_index layout), one 16-byte load per lane.
-    const int rg0 = (m0 >> 4) + wm * TM;
-    const int frag_k = 8 * (lane >> 4); // k offset of this lane's B fragment within a block
-    const int rg_last = (M - 1) >> 4; // groups past M feed unstored rows
-    const rsrc_t ra = make_rsrc(a.xt, (uint32_t)(rg_last + 1) * nblk * 2048);
-    uint32_t va[TM];
-#pragma unroll
-    for (int mi = 0; mi < TM; mi++) va[mi] = ((uint32_t)min(rg0 + mi, rg_last) * nblk * 1024 + lane * 8) * 2;
-    rsrc_t rs;
-    uint32_t vs[TM];
-    if (TYPE == kQ5_1) {
-        rs = make_rsrc(a.xsum, (uint32_t)M * nblk * 4);
-#pragma unroll
-        for (int mi = 0; mi < TM; mi++) vs[mi] = (uint32_t)(m0 + wm * TM * 16 + mi * 16 + 4 * (lane >> 4)) * nblk * 4;
-    }
-    auto load_a = [&](int st, AFrag<TM> &f) {
-        st = min(st, nstage - 1);
-#pragma unroll
-        for (int mi = 0; mi < TM; mi++) {
-#pragma unroll
-            for (int kb2 = 0; kb2 < 2; kb2++) {
-                const int kblk = kb_begin + min(2 * st + kb2, nb - 1);
-                f.hi[mi][kb2] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(ra, va[mi], kblk * 2048, 0));
-                f.lo[mi][kb2] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(ra, va[mi] + 1024, kblk * 2048, 0));
-                if (TYPE == kQ5_1) {
-                    // rows past M read zeros (outside the buffer) and are never stored
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        f.s[mi][kb2][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, vs[mi] + r * nblk * 4, kblk * 4, 0));
-                }
-            }
-        }
-    };
-
-    floatx4 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-    // Per block: p = x_hi . q, p += x_lo . q (MFMA), acc = fma(d, p, acc)
-    // (+ m * sum(x)).  KS blocks' partials are in flight together so each MFMA
-    // result is consumed several MFMAs after it issues; the FMAs still apply
-    // block 0 before block 1 for every output.
-    static_assert(KS == 1 || KS == 2, "one or two blocks in flight");
-    auto compute = [&](int st, int buf, const AFrag<TM> &f) {
-        const bool second = 2 * st + 1 < nb;
-#pragma unroll
-        for (int k0 = 0; k0 < 2; k0 += KS) {
-#pragma unroll
-            for (int g = 0; g < TN / NG; g++) {
-                half8_t fb[KS][NG];
-                float dsc[KS][NG], mn[KS][NG];
-                floatx4 p[KS][TM][NG];
-#pragma unroll
-                for (int kk = 0; kk < KS; kk++)
-#pragma unroll
-                    for (int n = 0; n < NG; n++) {
-                        int c = wn * TN * 16 + (g * NG + n) * 16 + (lane & 15);
-                        fb[kk][n] = *(const half8_t *)(&Bs[buf][c * LROW + (k0 + kk) * 32 + frag_k]);
-                        dsc[kk][n] = Ds[buf][c * 2 + k0 + kk];
-                        if (TYPE == kQ5_1) mn[kk][n] = Ms[buf][c * 2 + k0 + kk];
-                    }
-#pragma unroll
-                for (int kk = 0; kk < KS; kk++)
-#pragma unroll
-                    for (int mi = 0; mi < TM; mi++)
-#pragma unroll
-                        for (int n = 0; n < NG; n++)
-                            p[kk][mi][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.hi[mi][k0 + kk], fb[kk][n],
-                                                                                   floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-                for (int kk = 0; kk < KS; kk++)
-#pragma unroll
-                    for (int mi = 0; mi < TM; mi++)
-#pragma unroll
-                        for (int n = 0; n < NG; n++)
-                            p[kk][mi][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.lo[mi][k0 + kk], fb[kk][n],
-                                                                                   p[kk][mi][n], 0, 0, 0);
-#pragma unroll
-                for (int kk = 0; kk < KS; kk++) {
-                    // an odd block count's missing second block adds 0 * p (p is finite):
-                    // no branch inside the stage's straight-line code
-                    const bool live = k0 + kk == 0 || second;
-#pragma unroll
-                    for (int mi = 0; mi < TM; mi++)
-#pragma unroll
-                        for (int n = 0; n < NG; n++)
-#pragma unroll
-                            for (int r = 0; r < 4; r++) {
-                                float v = fmaf(live ? dsc[kk][n] : 0.f, p[kk][mi][n][r], acc[mi][g * NG + n][r]);
-                                if (TYPE == kQ5_1) v = fmaf(live ? mn[kk][n] : 0.f, f.s[mi][k0 + kk][r], v);
-                                acc[mi][g * NG + n][r] = v;
-                            }
-                }
-            }
-        }
-    };
-
-    // ---- software pipeline.  Ring of U = PD + 1 register slots: A fragments
-    // are loaded PD stages ahead, raw weight chunks PD + 1 stages ahead (they
-    // are decoded into LDS one stage before use).  The loop is unrolled by U
-    // so every ring index is a compile-time constant.
-    constexpr int U = PD + 1;
-    BChunk br[U][CPT];
-    AFrag<TM> fa[U];
-#pragma unroll
-    for (int j = 0; j < PD; j++) load_a(j, fa[j]);
-#pragma unroll
-    for (int j = 0; j <= PD; j++) load_b(j, br[j]);
-    store_b(0, br[0]);
-    __syncthreads();
-
-    // Stage s: compute it (LDS buffer s & 1, A slot s % U), decode stage
-    // s + 1 into the other buffer, refill the freed slots.  The loop runs
-    // whole groups of U stages only and the remainder follows it: a loop with
-    // exits inside its body would merge a half-advanced ring into the loop
-    // header, where the compiler would then drain every outstanding load.
-    auto stage = [&](auto jc, int s) {
-        constexpr int j = decltype(jc)::value;
-        load_a(s + PD, fa[(j + PD) % U]);
-        compute(s, s & 1, fa[j]);
-        store_b((s + 1) & 1, br[(j + 1) % U]);
-        load_b(s + PD + 1, br[j]);
-        __syncthreads();
-    };
-    const int ngroups = nstage / U;
-    int s0 = 0;
-    for (int g = 0; g < ngroups; g++, s0 += U) {
-        stage(std::integral_constant<int, 0>{}, s0);
-        if constexpr (U > 1) stage(std::integral_constant<int, 1 % U>{}, s0 + 1);
-        if constexpr (U > 2) stage(std::integral_constant<int, 2 % U>{}, s0 + 2);
-        if constexpr (U > 3) stage(std::integral_constant<int, 3 % U>{}, s0 + 3);
-        static_assert(U <= 4, "ring deeper than the unrolled group");
-    }
-    {
-        const int rem = nstage - s0;
-        if constexpr (U > 1) if (rem > 0) stage(std::integral_constant<int, 0>{}, s0);
-        if constexpr (U > 2) if (rem > 1) stage(std::integral_constant<int, 1 % U>{}, s0 + 1);
-        if constexpr (U > 3) if (rem > 2) stage(std::integral_constant<int, 2 % U>{}, s0 + 2);
-    }
-
-    // ---- epilogue.  Lane holds C[4*(lane/16) + r][lane % 16] of each 16x16 tile.
-    const int row_base = m0 + wm * TM * 16 + 4 * (lane >> 4);
-    if (MODE == kGemmStore) {
-        float *y = a.y + (size_t)z * M * a.ldy;
-        int seg, r0;
-        map_row<MODE, BN>(a, tile_n, 0, seg, r0); // segment and local row of the tile's first column
-        const QWeight &ws = a.seg[seg];
-        const int col0 = tile_n * BN;
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            int off = wn * TN * 16 + j * 16 + (lane & 15);
-            if (r0 + off >= ws.rows) continue;
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    int row = row_base + 16 * i + r;
-                    if (row < M) __builtin_nontemporal_store(acc[i][j][r], &y[(size_t)row * a.ldy + col0 + off]);
-                }
-        }
-    } else {
-        const int ld = a.seg[0].rows;
-        const int cbase = tile_n * (BN / 2);
-#pragma unroll
-        for (int pp = 0; pp < TN / 2; pp++) {
-            // N tiles 2pp (gate) and 2pp+1 (up) of this wave cover the same outputs
-            int col = cbase + ((wn * TN + 2 * pp) >> 1) * 16 + (lane & 15);
-            if (col >= ld) continue;
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    int row = row_base + 16 * i + r;
-                    if (row >= M) continue;
-                    // Kernels.SwiGlu (Kernels.cs:82-89): (g*u) * sigmoid(g).
-                    float g = acc[i][2 * pp][r], u = acc[i][2 * pp + 1][r];
-                    float gu = g * u;
-                    float e = expf(-g);
-                    float sg = 1.0f / (1.0f + e);
-                    float v = sg * gu;
-                    uint16_t hi, lo;
-                    split_f16(v, hi, lo);
-                    a.ot[xt_index(row, col, ld >> 5, 0)] = hi;
-                    a.ot[xt_index(row, col, ld >> 5, 1)] = lo;
-                }
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------
-// B-direct variant: the four waves sit side by side along N, each owning TN
-// weight tiles (16 rows each) that it streams from HBM straight into
-// registers and decodes there -- a tile slot is exactly the lane's B fragment
-// -- while the BM x 64 activation tile of a stage is loaded once per
-// workgroup into LDS and read by all four waves.  Per MFMA this moves half
-// the bytes through the vector-memory path and the LDS of the variant above
-// (whose B tile goes through LDS and whose A fragments come per wave from
-// L2).  The arithmetic per output is the same sequence of MFMAs and FMAs, so
-// the two variants agree bit for bit and either may serve any M.
+// B-direct: the waves sit side by side along N, each owning TN weight tiles
+// (16 rows each) that it streams from HBM straight into registers and decodes
+// there -- a tile slot is exactly the lane's B fragment -- while the BM x 64
+// activation tile of a stage is loaded once per workgroup into LDS and read by
+// all of them.
 //
 // FOLD: the workgroup walks every K-split range of its tile in order (the
 // grid has no split dimension), each range's chain from zero as a split
 // workgroup would run it, and keeps the ranges' sum in split order in a
 // second accumulator set; it stores that sum once instead of ksplit partials.
 //
-// NW: waves per workgroup, side by side along N (BN = 16 TN NW).  Twelve
-// waves share one activation tile three times as wide as four do: a third of
-// the activation loads and LDS stores per MFMA.  At 256 rows of the 3B
-// projections that gives 256 workgroups of 12 waves, one per CU and the same
-// three waves per SIMD as 768 workgroups of four (QKV 27.4 -> 26.2 us, O 20.0
-// -> 19.2, down 39.1 -> 36.2; cold weights).
+// NW: waves per workgroup, side by side along N (BN = 16 TN NW).  All of them
+// share one activation tile: the wider the workgroup, the fewer activation
+// loads and LDS stores per MFMA.
 template <int TYPE, int MODE, int TM, int TN, int PD, int OCC, bool FOLD = false, int NW = 4>
 __global__ __launch_bounds__(64 * NW, OCC) void gemm_bd_kernel(GemmArgs a, int mt, int nt, int gm)
 {
     constexpr int BM = 16 * TM, BN = 16 * TN * NW;
     constexpr int U = PD + 1; // weight register ring
     static_assert(!FOLD || MODE == kGemmStore, "folded K splits are a store-mode form");
-    static_assert(NW % 4 == 0, "whole groups of four waves");
     __shared__ __attribute__((aligned(16))) uint16_t As[2][TM * 4 * 512]; // [mi][block][part] operand tiles
 
-    // ---- tile of this workgroup (same order and K splits as gemm_q_kernel)
+    // ---- tile of this workgroup (per-XCD runs of a grouped order; K split z = whole runs of it)
     const int total = gridDim.x;
     const int per_xcd = total >> 3;
     const int L = blockIdx.x;
@@ -586,11 +202,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void gemm_bd_kernel(GemmArgs a, int m
     };
 
     // ---- weight loader: tile n of this wave is tile row wave * TN + n of the workgroup
-    // byte quants (see quant_rsrc), Q5_1 but in the 64 x 256 tile
-    constexpr bool BQ = TYPE == kQ8_0 || (TYPE == kQ5_1 && TM * TN < 16);
-    rsrc_t rq[TN], rd[TN], rh[TN];
+    constexpr bool BQ = kByteQuants<TYPE>;
+    rsrc_t rq[TN], rd[TN];
     int btile0[TN];
-    const uint32_t vq = (uint32_t)lane * (BQ ? 16 : 8), vd = 4 * (lane & 15), vh = 2 * lane;
+    const uint32_t vq = (uint32_t)lane * (BQ ? 16 : 8), vd = 4 * (lane & 15);
 #pragma unroll
     for (int n = 0; n < TN; n++) {
         const int t = wave * TN + n;
@@ -614,9 +229,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void gemm_bd_kernel(GemmArgs a, int m
         const QWeight &w = a.seg[seg];
         const int KP = tile_kpairs(w.cols), RG = tile_rows(w.rows);
         const uint32_t tiles = (uint32_t)RG * KP;
-        rq[n] = quant_rsrc<TYPE, BQ>(w, tiles);
+        rq[n] = quant_rsrc<TYPE>(w, tiles);
         rd[n] = make_rsrc(w.d, tiles * tile_d_bytes(TYPE));
-        if (TYPE == kQ5_1 && !BQ) rh[n] = make_rsrc(w.qh, tiles * 128);
         btile0[n] = __builtin_amdgcn_readfirstlane(min(rgw, RG - 1) * KP + (kb_begin >> 1));
     }
     auto load_b = [&](int st, BChunk (&br)[TN]) __attribute__((always_inline)) {
@@ -634,7 +248,6 @@ __global__ __launch_bounds__(64 * NW, OCC) void gemm_bd_kernel(GemmArgs a, int m
                 const uint2 dm = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rd[n], 2 * vd, tile * 128, 0));
                 br[n].d = dm.x;
                 br[n].m = dm.y;
-                if (!BQ) br[n].qh = __builtin_amdgcn_raw_buffer_load_b16(rh[n], vh, tile * 128, 0);
             } else {
                 br[n].d = __builtin_amdgcn_raw_buffer_load_b32(rd[n], vd, tile * 64, 0);
             }
@@ -694,7 +307,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void gemm_bd_kernel(GemmArgs a, int m
             float dv[TN], mv[TN];
 #pragma unroll
             for (int n = 0; n < TN; n++) {
-                bf[n] = decode_b_frag<TYPE, BQ>(br[n], bb);
+                bf[n] = decode_b_frag<TYPE>(br[n], bb);
                 dv[n] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, h2f((uint16_t)(bb ? br[n].d >> 16 : br[n].d))) & live);
                 if (TYPE == kQ5_1)
                     mv[n] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, h2f((uint16_t)(bb ? br[n].m >> 16 : br[n].m))) & live);
@@ -740,8 +353,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void gemm_bd_kernel(GemmArgs a, int m
     // ---- pipeline: weights U stages ahead in a register ring; activations
     // loaded UA stages ahead into a register ring (stage t in slot t % UA)
     // and copied to LDS (double buffered) by the stage before their own.
-    // Whole groups of U stages in the loop, the remainder after it (see
-    // gemm_q_kernel).  The prologue issues its loads in the loop's order
+    // Whole groups of U stages in the loop, the remainder after it: a loop
+    // with exits inside its body would merge a half-advanced ring into the
+    // loop header, where the compiler would then drain every outstanding load.
+    // The prologue issues its loads in the loop's order
     // (activations of stage t + 1, then weights of stage t) so the compiler's
     // wait counts at the loop head, merged over entry and back edge, stay
     // those of the loop.
@@ -903,7 +518,7 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(GemmArgs a, int ngr
     if (TYPE == kQ5_1) rs = make_rsrc(a.xsum, (uint32_t)M * nblk * 4);
 
     // weights: tile n of this wave
-    constexpr bool BQ = TYPE != kQ4_0; // byte quants (see quant_rsrc)
+    constexpr bool BQ = kByteQuants<TYPE>;
     rsrc_t rq[TN], rd[TN];
     int btile0[TN];
     int seg_store = 0, start_store = 0;
@@ -929,7 +544,7 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(GemmArgs a, int ngr
         const QWeight &wt = a.seg[seg];
         const int KP = tile_kpairs(wt.cols), RG = tile_rows(wt.rows);
         const uint32_t tiles = (uint32_t)RG * KP;
-        rq[n] = quant_rsrc<TYPE, BQ>(wt, tiles);
+        rq[n] = quant_rsrc<TYPE>(wt, tiles);
         rd[n] = make_rsrc(wt.d, tiles * tile_d_bytes(TYPE));
         btile0[n] = __builtin_amdgcn_readfirstlane(min(rgw, RG - 1) * KP + (kb_begin >> 1));
     }
@@ -997,7 +612,7 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(GemmArgs a, int ngr
             if (TYPE == kQ5_1) xs4 = *(const floatx4 *)&Xs[buf][(sl * 2 + bb) * 16 + 4 * (lane >> 4)];
 #pragma unroll
             for (int n = 0; n < TN; n++) {
-                const half8_t bf = decode_b_frag<TYPE, BQ>(br[n], bb);
+                const half8_t bf = decode_b_frag<TYPE>(br[n], bb);
                 const float dv = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, h2f((uint16_t)(bb ? br[n].d >> 16 : br[n].d))) & live);
                 float mv = 0.f;
                 if (TYPE == kQ5_1)
@@ -1134,63 +749,92 @@ static hipError_t launch_bd(const GemmArgs &a, hipStream_t s, int gm_cap = 8)
     return hipGetLastError();
 }
 
-template <int TYPE, int MODE, int WM, int WN, int TM, int TN, int PD, int KS, int OCC>
-static hipError_t launch_cfg(const GemmArgs &a, hipStream_t s)
-{
-    constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
-    int mt = (a.M + BM - 1) / BM;
-    int ncols;
-    if (MODE == kGemmSwiGlu) {
-        ncols = (a.seg[0].rows + BN / 2 - 1) / (BN / 2);
-    } else {
-        int ntot = 0;
-        for (int i = 0; i < a.nseg; i++) ntot += a.seg[i].rows;
-        ncols = (ntot + BN - 1) / BN;
-    }
-    int gm = mt <= 8 ? mt : 8;
-    int tiles = mt * ncols;
-    int grid = ((tiles + 7) & ~7) * a.ksplit;
-    launch_stamped(a.ev_start, a.ev_stop, gemm_q_kernel<TYPE, MODE, WM, WN, TM, TN, PD, KS, OCC>, dim3(grid), dim3(256), 0,
-                   s, a, mt, ncols, gm);
-    return hipGetLastError();
-}
+// Tile choice.  It only changes which rows and columns share a workgroup,
+// never a result bit.  What bounds these grids below ~700 rows is the busiest
+// compute unit: each wave's K stage costs about the same whatever runs beside
+// it (its MFMAs, the scale FMAs and the decode share one issue port), every
+// workgroup stages its own copy of the activation tile, and a second workgroup
+// on a few of the 256 compute units doubles the launch.  So the workgroup is
+// made just wide enough that the grid is one round -- one workgroup per
+// compute unit, all of its waves sharing one activation tile -- and no wider
+// (a wave's share grows with the width).  Cold weights, 3B projections, in us,
+// four-wave 32 x 128 tiles (225..256 rows: twelve-wave) against these:
+//   Q8_0 QKV     32 rows 13.1 -> 9.4    64 13.3 -> 11.8   96 17.1 -> 14.6
+//               160 rows 18.0 -> 16.9  224 23.7 -> 21.6  320 33.3 -> 29.4
+//               512 rows 46.9 -> 44.0  640 (64 x 256) 55.5 -> 52.2
+//   Q5_1 down    32 rows 23.5 -> 15.8  128 33.5 -> 26.1  320 57.6 -> 52.2
+//               640 rows 111.9 -> 95.3, 1500 266 -> 232, 4528 665 -> 634
+//   Q8_0 SwiGLU  32 rows 29.2 -> 24.7   48 35.0 -> 25.0   96 35.8 -> 29.4
+//               128 rows 46.6 -> 35.9  192 62.1 -> 51.8  256 74.2 -> 69.7
+//               320 rows 89.5 -> 83.4  448 117 -> 101
+constexpr int kCUs = 256;
 
 template <int TYPE, int MODE>
 static hipError_t launch_mode(const GemmArgs &a, hipStream_t s)
 {
-    // Shape choice by M only changes which rows share a tile, never a result bit.
-    // Measured on MI355X (3B shapes, Q8_0): small batches take B-direct
-    // 32 x 128 tiles (4-5 % ahead of dequant-in-LDS 64 x 64 tiles on the
-    // store shapes), large batches B-direct 64 x 256 tiles.  B-direct needs
-    // the store-mode segments to split on 256-row boundaries.
-    bool bd_ok = true;
-    for (int i = 0; i + 1 < a.nseg; i++) bd_ok = bd_ok && a.seg[i].rows % 256 == 0;
     // One row group (the reasoning decider's rows, short branches): one wave
     // per weight row group, 1.5-2x the B-direct kernel there (12 rows of the
     // Q5_1 3B shape: 2.1 against 3.6 ms of GEMM per step)
     if (a.M <= 16) return launch_skinny<TYPE, MODE, 4, 8>(a, s);
-    if (a.M <= 512) {
-        // SwiGLU (9216 rows at 256 tokens: 1152 workgroups): built for five
-        // resident workgroups per CU (80 VGPRs, six fit) so they all run in
-        // one round -- 3 % ahead alone, 0.15 % of a prefill step in the
-        // model; the store shapes lose 4-5 % that way.  Groups of 4 M tiles
-        // in the tile order: 8 % faster than 8 at 256 tokens (the store
-        // shapes are indifferent)
-        if (MODE == kGemmSwiGlu) return launch_bd<TYPE, MODE, 2, 2, 1, 5>(a, s, 4);
-        // 225..256 rows: 12-wave workgroups (one per CU at the 3B projection
-        // shapes, three waves per SIMD), 4-8 % ahead of 4-wave ones.  Fewer
-        // rows would leave CUs idle, more would need a second round.
-        if constexpr (MODE == kGemmStore)
-            if (bd_ok && a.M > 224 && a.M <= 256) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 12>(a, s);
-        if (bd_ok) return launch_bd<TYPE, MODE, 2, 2, 1, 4>(a, s);
-        return launch_cfg<TYPE, MODE, 4, 1, 1, 4, 2, 2, 2>(a, s);
+    int tcols; // 16-wide tile columns of the output (gate and up both count)
+    if (MODE == kGemmSwiGlu) {
+        tcols = 2 * (a.seg[0].rows / 16);
+    } else {
+        int ntot = 0;
+        for (int i = 0; i < a.nseg; i++) ntot += a.seg[i].rows;
+        tcols = (ntot + 15) / 16;
     }
-    if (bd_ok) {
-        if constexpr (MODE == kGemmStore && TYPE != kQ5_1)
-            if (a.fold) return launch_bd<TYPE, MODE, 4, 4, 1, 2, true>(a, s);
-        return launch_bd<TYPE, MODE, 4, 4, 1, 2>(a, s);
+    // workgroups of a grid of 16 tm x 16 tn nw tiles
+    auto wgs = [&](int tm, int tn, int nw) {
+        return (long)((a.M + 16 * tm - 1) / (16 * tm)) * ((tcols + tn * nw - 1) / (tn * nw)) * a.ksplit;
+    };
+    if constexpr (MODE == kGemmSwiGlu) {
+        if (a.M <= 512) {
+            if (wgs(1, 2, 8) <= kCUs) return launch_bd<TYPE, MODE, 1, 2, 1, 1, false, 8>(a, s, 4);
+            if (wgs(2, 2, 8) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 8>(a, s, 4);
+            if (wgs(2, 2, 10) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 10>(a, s, 4);
+            if (wgs(2, 2, 12) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 12>(a, s, 4);
+            if constexpr (TYPE != kQ5_1) {
+                // (four waves per SIMD leave 128 registers: Q5_1's block sums do not fit, 74 -> 98 us at 192 rows)
+                if (wgs(2, 2, 14) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 14>(a, s, 4);
+                if (wgs(2, 2, 16) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 16>(a, s, 4);
+            }
+            // 64-row tiles (half the decode per MFMA) where their grid nearly
+            // fills the round; nine waves only when the last tile is more than
+            // half full (208 rows of Q5_1: 76 -> 86 us)
+            long g = wgs(4, 2, 9);
+            if (g <= kCUs && g > kCUs * 7 / 8 && (a.M - 1) % 64 >= 32) return launch_bd<TYPE, MODE, 4, 2, 1, 1, false, 9>(a, s);
+            g = wgs(4, 2, 12);
+            if (g <= kCUs && g > kCUs * 7 / 8) return launch_bd<TYPE, MODE, 4, 2, 1, 1, false, 12>(a, s);
+            g = wgs(4, 2, 8);
+            if (g <= 2 * kCUs && g > kCUs * 3 / 2) return launch_bd<TYPE, MODE, 4, 2, 1, 1, false, 8>(a, s); // two per CU
+            // no width fits: four-wave tiles built for five resident
+            // workgroups per CU (80 VGPRs), in groups of 4 M tiles
+            return launch_bd<TYPE, MODE, 2, 2, 1, 5>(a, s, 4);
+        }
+    } else if (a.M <= 512) {
+        // (up to 2.25 of these short workgroups per CU beat wider ones: 48 rows of QKV, Q8_0 11.7 -> 10.8 us, Q4_0 12.4 -> 11.3)
+        if (wgs(1, 1, 4) <= kCUs * 9 / 4) return launch_bd<TYPE, MODE, 1, 1, 1, 4>(a, s);
+        if (wgs(2, 1, 8) <= kCUs) return launch_bd<TYPE, MODE, 2, 1, 1, 1, false, 8>(a, s);
+        if (wgs(2, 1, 12) <= kCUs) return launch_bd<TYPE, MODE, 2, 1, 1, 1, false, 12>(a, s);
+        if (wgs(2, 2, 8) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 8>(a, s);
+        if (wgs(2, 2, 12) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 12>(a, s);
+        // two or three per CU; Q5_1's second FMA per output favours the taller tile (512 rows of QKV 68.3 -> 55.9 us)
+        if constexpr (TYPE == kQ5_1) return launch_bd<TYPE, MODE, 4, 1, 1, 1, false, 8>(a, s);
+        return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 8>(a, s);
     }
-    return launch_cfg<TYPE, MODE, 4, 1, 2, 8, 1, 1, 2>(a, s);
+    // Large batches.  Four-wave 64 x 256 tiles keep 16 tiles per wave, and
+    // with them Q5_1 has no registers for its byte quants: eight waves of 64 x
+    // 32 there at every size.  A four-wave tile must lie in one segment.
+    bool one_seg = true;
+    if (MODE == kGemmStore)
+        for (int i = 0; i + 1 < a.nseg; i++) one_seg = one_seg && a.seg[i].rows % 256 == 0;
+    if constexpr (MODE == kGemmStore && TYPE != kQ5_1)
+        if (a.fold) return launch_bd<TYPE, MODE, 4, 4, 1, 2, true>(a, s);
+    if (TYPE == kQ5_1 || !one_seg || (MODE == kGemmStore && wgs(4, 2, 8) <= 2 * kCUs))
+        return launch_bd<TYPE, MODE, 4, 2, 1, 1, false, 8>(a, s);
+    if constexpr (TYPE != kQ5_1) return launch_bd<TYPE, MODE, 4, 4, 1, 2>(a, s);
+    return hipErrorInvalidValue; // not reached
 }
 
 template <int TYPE>
