@@ -261,8 +261,29 @@ constexpr int kAttnTileTokens = 32;
 struct AttnTile {
     int32_t t0, n, shared_lo, shared_hi, segment, slot0, pad0, pad1;
 };
+// Logical key blocks (of 64) per partition: a tile's online softmax restarts
+// at every partition and the partitions merge in ascending order.  512 keys
+// are the largest power of two that still spreads a 4096-token context over
+// the GPU for a handful of queries; the merge costs a tile ~3 % of a
+// partition's own time.
+constexpr int kAttnPartBlocks = 8;
+constexpr int kAttnPartFloats = 64 + 32 * 128; // one tile and head's partial: 32 maxima, 32 sums, 32 x 128 outputs
+// How a pass's attention is cut into workgroups: ds of them per (tile, KV
+// head) share the output dims, and with run_blocks > 0 every run of that many
+// blocks (whole partitions) is a workgroup of its own whose partials
+// attn_merge_kernel merges.  No choice changes a result bit.
+struct AttnSchedule {
+    int ds = 1;
+    int run_blocks = 0; // 0: one workgroup walks all blocks of its tile
+    int n_parts = 1;
+    size_t floats = 0;  // workspace of the partials
+};
+AttnSchedule attn_schedule(int n_tiles, int n_heads, int group, int max_blocks, double total_blocks);
 struct AttnArgs {
     int n_tiles = 0, n_heads = 0, group = 4, hd = 128;
+    AttnSchedule sched;
+    float *part = nullptr; // sched.floats floats when the blocks are split
+    int run_blocks = 0, n_parts = 1; // filled by launch_attn_tree from sched
     const AttnTile *tiles = nullptr;
     const float *q = nullptr; // [T][qdim]
     const uint16_t *kp = nullptr, *vp = nullptr; // pair shadows, layer base [kvh][cap][hi, lo][hd]

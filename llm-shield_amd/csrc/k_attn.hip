@@ -31,11 +31,23 @@
 //   O^T (128 x 32) += V^T (128 x 64) . P^T (64 x 32)      48 MFMAs per 64 keys,
 //                     keys taken in the order the S^T fragments hold them
 //
+// Partitions.  The blocks form partitions of kAttnPartBlocks (512 logical
+// keys), each its own online softmax from scratch, and the partitions' (max,
+// sum, o) are merged in ascending order: a rule on the logical key index alone,
+// so a query's arithmetic still does not depend on what runs beside it, and a
+// partition may run in any workgroup.  A pass whose tiles and heads fill the
+// GPU walks all partitions of a tile in one workgroup and merges as it goes; a
+// few queries over a long context (a question or a set of options over a cached
+// policy) give each run of partitions its own workgroup, leave the partials in
+// memory and merge them in attn_merge_kernel (attn_schedule has the choice and
+// its measurements).
+//
 // Decode kernel (attn_decode_kernel): one query per head, split over chunks
 // of 64 logical keys per KV head; the chunks are combined in ascending order
 // by the consumer, the O projection's GEMV, while it stages its input.
 #include "jev_dev.h"
 
+#include <cmath>
 #include <type_traits>
 
 namespace jev {
@@ -104,8 +116,7 @@ __device__ __forceinline__ half8_t cat4(uint2 a, uint2 b)
 }
 } // namespace
 
-// DS = 2 or 4 (grids smaller than the GPU): DS workgroups per tile and KV
-// head (blockIdx.z); each stages the blocks and computes the scores and
+// DS = 2 or 4 (few tiles): DS workgroups per tile and KV head; each stages the blocks and computes the scores and
 // softmax (the same instructions on the same data) and accumulates 128 / DS
 // of the output dims.  Every output is the same chain of MFMAs either way.
 //
@@ -118,7 +129,11 @@ __device__ __forceinline__ half8_t cat4(uint2 a, uint2 b)
 //         half of block b's softmax (mask, running max, exponentials).
 // The operations and their order per output are those of the plain sequence
 // S(b), P V(b - 1), softmax(b), rescale, so the bits do not depend on it.
-template <int DS>
+//
+// SPLIT: blockIdx.z also counts runs of a.run_blocks blocks (whole
+// partitions); the workgroup walks its run and stores each partition's (max,
+// sum, o) instead of merging them.
+template <int DS, bool SPLIT>
 __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
 {
     constexpr int ND = 4 / DS; // 32-dim output tiles per wave
@@ -138,7 +153,7 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
     const int hsets = (a.group + 3) >> 2;
     const int kvh = blockIdx.x / hsets;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int dh = DS > 1 ? (int)blockIdx.z : 0; // output dims 128 / DS * dh ..
+    const int dh = DS > 1 ? (int)blockIdx.z % DS : 0; // output dims 128 / DS * dh ..
     const int g = lane >> 5, col = lane & 31;
     const int hl = (blockIdx.x % hsets) * 4 + wave; // query head within the group
     const bool head_ok = hl < a.group;              // wave-uniform
@@ -152,7 +167,11 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
     const int my_limit = q_ok ? n_sh + (tile.slot0 + col - tile.segment + 1) : 1;
     const int min_limit = n_sh + (tile.slot0 - tile.segment + 1); // the tile's first query
     const int max_limit = n_sh + (tile.slot0 + tile.n - 1 - tile.segment + 1);
-    const int nblocks = (max_limit + KB - 1) / KB;
+    const int nblocks_all = (max_limit + KB - 1) / KB;
+    // this workgroup's blocks [b0, b1); b0 is a multiple of kAttnPartBlocks
+    const int b0 = SPLIT ? (int)blockIdx.z / DS * a.run_blocks : 0;
+    if (SPLIT && b0 >= nblocks_all) return; // a shorter tile
+    const int b1 = SPLIT ? min(nblocks_all, b0 + a.run_blocks) : nblocks_all;
     auto slot_of = [&](int kl) { return kl < n_sh ? tile.shared_lo + kl : tile.segment + (kl - n_sh); };
 
     // Staging: wave w's load i moves LDS chunks (8 w + i) * 64 + lane, i.e.
@@ -195,7 +214,7 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
     };
     const rsrc_t kpb = make_rsrc(a.kp + (size_t)kvh * a.cap * 256, (uint32_t)a.cap * 512);
     const rsrc_t vpb = make_rsrc(a.vp + (size_t)kvh * a.cap * 256, (uint32_t)a.cap * 512);
-    stage(0, kpb, Ks0); // in flight while Q is read
+    stage(b0, kpb, Ks0); // in flight while Q is read
 
     // Q^T fragments: dims 16 c + 8 g .. + 7 of this lane's query, scaled by
     // 1/sqrt(head_dim) * log2 e (scores come out in log2 units), as pairs.
@@ -249,7 +268,8 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
     for (int d = 0; d < ND; d++)
 #pragma unroll
         for (int j = 0; j < 16; j++) o[d][j] = 0.f;
-    float m_run = -INFINITY, l_run = 0.f; // running max in log2 units
+    float m_run = -INFINITY, l_run = 0.f; // running max (log2 units) and sum of the partition
+    float m_old = -INFINITY;              // the running max before the block in ex
     float alpha = 0.f;                    // exp2(previous max - new max) of the block in ex
     floatx16 sc[2];                       // S^T of the block being scored
     floatx16 ex[2];                       // exp2(s - max) of the block in the softmax
@@ -351,9 +371,14 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
         }
         if (k == BPERM) bmax_o = __shfl_xor(bmax, 32, 64);
         if (k == MNEW) {
-            m_new = fmaxf(m_run, fmaxf(bmax, bmax_o));
-            alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+            // a partition's first block starts from scratch: alpha is 0
+            m_old = m_run;
+            const float mp = b % kAttnPartBlocks == 0 ? -INFINITY : m_run;
+            m_new = fmaxf(mp, fmaxf(bmax, bmax_o));
             m_run = m_new;
+            // a query that sees nothing of its partition yet: exponentials of -inf - 0
+            if constexpr (decltype(masked)::value) m_new = m_new == -INFINITY ? 0.f : m_new;
+            alpha = __builtin_amdgcn_exp2f(mp - m_new);
         }
         if (k >= EXP0 && k < EXP0 + 32 / PER) {
 #pragma unroll
@@ -400,39 +425,91 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
     // block b reaches past the tile's first query: its scores need the mask
     auto tail = [&](int b) { return (b + 1) * KB > min_limit; };
 
-    // Block 0: staged K(1) and V(0), S(0) and its softmax's first half.
-    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): this thread's K(0) has landed
+    // The finished partitions' merge, in accumulation registers (one workgroup
+    // for the whole tile) or in memory (SPLIT).
+    constexpr bool MERGE = !SPLIT;
+    floatx16 ot[MERGE ? ND : 1];
+    float m_tot = -INFINITY, l_tot = 0.f;
+    if constexpr (MERGE) {
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+            ot[d] = floatx16{};
+            asm volatile("" : "+a"(ot[d]));
+        }
+    }
+    // Ends partition p, whose max is m and whose sum and output are l_run and
+    // o: (M, L, O) = the merge of (M, L, O) and (m, l, o) at their larger max.
+    // The first partition merges into nothing (factors 0 and 1), one that a
+    // query does not reach leaves its result as it is (factors 1 and 0).
+    auto end_part = [&](int p, float m) __attribute__((always_inline)) {
+        if constexpr (MERGE) {
+            const float mn = fmaxf(m_tot, m);
+            const float fo = __builtin_amdgcn_exp2f(m_tot - mn), fp = __builtin_amdgcn_exp2f(m - mn);
+            l_tot = fmaf(l_run, fp, l_tot * fo);
+            m_tot = mn;
+#pragma unroll
+            for (int d = 0; d < ND; d++) {
+#pragma unroll
+                for (int j = 0; j < 16; j++) ot[d][j] = fmaf(o[d][j], fp, ot[d][j] * fo);
+                asm volatile("" : "+a"(ot[d]));
+            }
+        } else if (q_ok) {
+            // [tile][head][partition]: the 32 queries' maxima, their sums, then
+            // o as [dim / 4][query][4] (32 lanes store 512 contiguous bytes)
+            float *pp = a.part + (((size_t)(a.n_tiles - 1 - (int)blockIdx.y) * a.n_heads + head) * a.n_parts + p) * kAttnPartFloats;
+            if (dh == 0 && g == 0) {
+                pp[col] = m;
+                pp[32 + col] = l_run;
+            }
+#pragma unroll
+            for (int d = 0; d < ND; d++)
+#pragma unroll
+                for (int jq = 0; jq < 4; jq++) {
+                    const int k4 = 8 * (ND * dh + d) + 2 * jq + g;
+                    *(float4 *)(pp + 64 + (k4 * 32 + col) * 4) =
+                        make_float4(o[d][4 * jq], o[d][4 * jq + 1], o[d][4 * jq + 2], o[d][4 * jq + 3]);
+                }
+        }
+        // o itself is left: the next partition's first block rescales it by 0
+    };
+
+    // First block: staged K(b0 + 1) and V(b0), S(b0) and its softmax's first half.
+    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): this thread's K(b0) has landed
     __syncthreads();                    // everyone's
-    if (nblocks > 1) stage(1, kpb, Ks1);
-    stage(0, vpb, Vs0);
+    if (b1 - b0 > 1) stage(b0 + 1, kpb, Ks1);
+    stage(b0, vpb, Vs0);
     // A wave past the group's last head (group not a multiple of 4) computes
     // its clamped head's rows like the others and stores nothing: no branch
     // around the block loop, so every block keeps o, sc and ex in place.
     scores(0, none);
-    if (tail(0)) {
+    if (tail(b0)) {
 #pragma unroll
-        for (int k = 0; k < NS1; k++) soft1(k, 0, Masked{});
+        for (int k = 0; k < NS1; k++) soft1(k, b0, Masked{});
     } else {
 #pragma unroll
-        for (int k = 0; k < NS1; k++) soft1(k, 0, Plain{});
+        for (int k = 0; k < NS1; k++) soft1(k, b0, Plain{});
     }
-    // Block b >= 1: K(b) in buffer b % 2, V(b - 1) in the other; K(b + 1) and
-    // V(b) are staged while A(b) and B(b) run.
+    // Block b > b0 (b0 is even): K(b) in buffer b % 2, V(b - 1) in the other;
+    // K(b + 1) and V(b) are staged while A(b) and B(b) run.
     auto step = [&](int b, uint32_t kb, uint32_t vb, uint4 *Kn, uint4 *Vn, auto masked) __attribute__((always_inline)) {
         __builtin_amdgcn_s_waitcnt(0x0F70); // this thread's K(b) and V(b - 1) have landed
         __syncthreads();                    // everyone's; K(b - 1) and V(b - 2) are free again
-        if (b + 1 < nblocks) stage(b + 1, kpb, Kn);
+        if (b + 1 < b1) stage(b + 1, kpb, Kn);
         stage(b, vpb, Vn);
         __builtin_amdgcn_sched_barrier(0);
         scores(kb, soft2);
         pv(vb, [&](int k) __attribute__((always_inline)) { soft1(k, b, masked); });
     };
-    for (int b = 1; b < nblocks; b += 2) {
+    // block b is the first of a partition: the one before it is complete in o
+    // once P V(b - 1) has run, which is before step b + 1
+    auto opens = [&](int b) { return b > b0 && b % kAttnPartBlocks == 0; };
+    for (int b = b0 + 1; b < b1; b += 2) {
+        if (opens(b - 1)) end_part((b - 1) / kAttnPartBlocks - 1, m_old);
         if (tail(b))
             step(b, KBUF, 0, Ks0, Vs1, Masked{});
         else
             step(b, KBUF, 0, Ks0, Vs1, Plain{});
-        if (b + 1 < nblocks) {
+        if (b + 1 < b1) {
             if (tail(b + 1))
                 step(b + 1, 0, KBUF, Ks1, Vs0, Masked{});
             else
@@ -440,12 +517,25 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
         }
     }
     // The last block's second softmax half and P V.
+    if (opens(b1 - 1)) end_part((b1 - 1) / kAttnPartBlocks - 1, m_old);
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 48; k++) soft2(k);
-    pv(((nblocks - 1) & 1) ? KBUF : 0, none);
+    pv(((b1 - 1) & 1) ? KBUF : 0, none);
 
+    if constexpr (SPLIT) {
+        end_part((b1 - 1) / kAttnPartBlocks, m_run);
+        return;
+    }
+    if (b1 > kAttnPartBlocks) { // several partitions: their merge
+        end_part(0, m_run);
+        if constexpr (MERGE) {
+#pragma unroll
+            for (int d = 0; d < ND; d++) o[d] = ot[d];
+        }
+        l_run = l_tot;
+    }
     if (q_ok) {
         // o[d][j] is dim 32 (ND dh + d) + 8 (j / 4) + 4 g + j % 4: four
         // consecutive k, one 8-byte store per part
@@ -465,23 +555,128 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
     }
 }
 
-hipError_t launch_attn_tree(const AttnArgs &a, hipStream_t s)
+// The partitions of a split pass merged in ascending order, with
+// attn_tree_kernel's own operations per output, then normalised and written as
+// it writes them.  One workgroup per (head, tile); wave w takes dims 32 w ..,
+// lane as in attn_tree_kernel (query lane % 32, dims 8 jq + 4 (lane / 32) ..).
+// Bound by reading the partials once.
+__global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a)
 {
+    const int head = blockIdx.x, ti = blockIdx.y;
+    const AttnTile tile = a.tiles[ti];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 5, col = lane & 31;
+    if (col >= tile.n) return;
+    const int max_limit = (tile.shared_hi - tile.shared_lo) + (tile.slot0 + tile.n - 1 - tile.segment + 1);
+    const int np = (max_limit + KB * kAttnPartBlocks - 1) / (KB * kAttnPartBlocks);
+    const float *pp = a.part + ((size_t)ti * a.n_heads + head) * a.n_parts * kAttnPartFloats;
+    float m_tot = -INFINITY, l_tot = 0.f;
+    float4 o[4];
+#pragma unroll
+    for (int jq = 0; jq < 4; jq++) o[jq] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int p = 0; p < np; p++, pp += kAttnPartFloats) {
+        const float m = pp[col], l = pp[32 + col];
+        float4 v[4];
+#pragma unroll
+        for (int jq = 0; jq < 4; jq++) v[jq] = *(const float4 *)(pp + 64 + ((8 * wave + 2 * jq + g) * 32 + col) * 4);
+        const float mn = fmaxf(m_tot, m);
+        const float fo = __builtin_amdgcn_exp2f(m_tot - mn), fp = __builtin_amdgcn_exp2f(m - mn);
+        l_tot = fmaf(l, fp, l_tot * fo);
+        m_tot = mn;
+#pragma unroll
+        for (int jq = 0; jq < 4; jq++) {
+            o[jq].x = fmaf(v[jq].x, fp, o[jq].x * fo);
+            o[jq].y = fmaf(v[jq].y, fp, o[jq].y * fo);
+            o[jq].z = fmaf(v[jq].z, fp, o[jq].z * fo);
+            o[jq].w = fmaf(v[jq].w, fp, o[jq].w * fo);
+        }
+    }
+    const float inv = 1.0f / l_tot;
+    const int t = tile.t0 + col, nblk = a.n_heads * 4;
+#pragma unroll
+    for (int jq = 0; jq < 4; jq++) {
+        const int k = head * 128 + 32 * wave + 8 * jq + 4 * g;
+        uint2 hv, lv;
+        split4(make_float4(o[jq].x * inv, o[jq].y * inv, o[jq].z * inv, o[jq].w * inv), hv, lv);
+        *(uint2 *)(a.ot + xt_index(t, k, nblk, 0)) = hv;
+        *(uint2 *)(a.ot + xt_index(t, k, nblk, 1)) = lv;
+    }
+}
+
+// The schedule is the cheapest of a small model of the launch: a workgroup
+// takes ~5 us to start and end, and per block of 64 keys 2.4 us (ds 1), 1.9
+// (ds 2: the scores are computed twice, P V half each) or 1.65 (ds 4); one
+// workgroup (128 KiB of LDS) runs per compute unit; a split pass pays the merge
+// launch and writes and reads its partials (~4 TB/s).  Measured (32 / 8 heads,
+// us per layer, one workgroup per tile and head group with the grid's ds
+// against this choice): 30 tokens over 4096 cached 106 -> 27, over 1100 33 ->
+// 21; 300 over 4096 124 -> 79, over 2000 67 -> 47; 5 options of 13 over 2000 57
+// -> 29; 9 options of 48 over 4096 250 (two rounds of ds 2) -> 141 (one of ds
+// 1); a 4096-token prompt's own tiles stay whole.
+AttnSchedule attn_schedule(int n_tiles, int n_heads, int group, int max_blocks, double total_blocks)
+{
+    constexpr int kCUs = 256;
+    constexpr double kStart = 5.0, kBlock[3] = {2.4, 1.9, 1.65}, kMerge = 4.0, kBytesPerUs = 4.0e6;
+    const double wide = (double)(n_heads / group) * ((group + 3) / 4); // workgroups per tile
+    AttnSchedule best;
+    best.n_parts = (max_blocks + kAttnPartBlocks - 1) / kAttnPartBlocks;
+    const size_t floats = (size_t)n_tiles * n_heads * best.n_parts * kAttnPartFloats;
+    double best_us = 1e30;
+    // jobs of at most `longest` blocks, `avg` blocks per compute unit in all:
+    // a second round starts when the work does not fit the first
+    auto blocks = [](double jobs, double longest, double avg) {
+        return jobs <= kCUs || avg <= 0.9 * longest ? longest : avg + 0.6 * longest;
+    };
+    for (int i = 0; i < 3; i++) {
+        const int ds = 1 << i;
+        const double avg = total_blocks * wide * ds / kCUs;
+        double jobs = n_tiles * wide * ds;
+        double us = blocks(jobs, max_blocks, avg) * kBlock[i] + kStart * std::ceil(jobs / kCUs);
+        if (us < best_us) {
+            best_us = us;
+            best.ds = ds;
+            best.run_blocks = 0;
+        }
+        if (best.n_parts < 2 || floats > ((size_t)1 << 27)) continue;
+        for (int run = kAttnPartBlocks; run < max_blocks; run *= 2) {
+            jobs = (total_blocks / run + 0.5 * n_tiles) * wide * ds; // half a run left over per tile
+            us = blocks(jobs, run, avg) * kBlock[i] + kStart * std::ceil(jobs / kCUs) + kMerge + 8.0 * floats / kBytesPerUs;
+            if (us < best_us) {
+                best_us = us;
+                best.ds = ds;
+                best.run_blocks = run;
+            }
+        }
+    }
+    best.floats = best.run_blocks > 0 ? floats : 0;
+    return best;
+}
+
+hipError_t launch_attn_tree(const AttnArgs &args, hipStream_t s)
+{
+    AttnArgs a = args;
     if (a.n_tiles <= 0) return hipSuccess;
     // cap * 512 bytes per KV head is a buffer resource's 32-bit extent (2^32
     // itself would wrap to an empty resource)
     if (a.hd != 128 || a.group < 1 || a.n_tiles > 65535 || !a.kp || !a.vp || a.cap <= 0 || a.cap >= (1 << 23))
         return hipErrorInvalidValue;
+    const AttnSchedule &c = a.sched;
+    if (c.run_blocks % kAttnPartBlocks != 0 || c.n_parts < 1 || (c.run_blocks > 0 && !a.part)) return hipErrorInvalidValue;
+    a.run_blocks = c.run_blocks;
+    a.n_parts = c.n_parts;
     const int n_kv = a.n_heads / a.group, hsets = (a.group + 3) / 4;
-    const dim3 grid(n_kv * hsets, a.n_tiles);
-    // fewer workgroups than compute units: the output dims split over two or four
-    const long wgs = (long)grid.x * grid.y;
-    if (wgs <= 64)
-        launch_stamped(a.ev_start, a.ev_stop, attn_tree_kernel<4>, dim3(grid.x, grid.y, 4), dim3(256), 0, s, a);
-    else if (wgs < 256)
-        launch_stamped(a.ev_start, a.ev_stop, attn_tree_kernel<2>, dim3(grid.x, grid.y, 2), dim3(256), 0, s, a);
-    else
-        launch_stamped(a.ev_start, a.ev_stop, attn_tree_kernel<1>, grid, dim3(256), 0, s, a);
+    const int runs = c.run_blocks > 0 ? (c.n_parts * kAttnPartBlocks + c.run_blocks - 1) / c.run_blocks : 1;
+    const dim3 grid(n_kv * hsets, a.n_tiles, c.ds * runs);
+    auto launch = [&](auto kernel) { launch_stamped(a.ev_start, a.ev_stop, kernel, grid, dim3(256), 0, s, a); };
+    if (c.run_blocks > 0) {
+        if (c.ds == 4) launch(attn_tree_kernel<4, true>);
+        else if (c.ds == 2) launch(attn_tree_kernel<2, true>);
+        else launch(attn_tree_kernel<1, true>);
+        hipLaunchKernelGGL(attn_merge_kernel, dim3(a.n_heads, a.n_tiles), dim3(256), 0, s, a);
+    } else {
+        if (c.ds == 4) launch(attn_tree_kernel<4, false>);
+        else if (c.ds == 2) launch(attn_tree_kernel<2, false>);
+        else launch(attn_tree_kernel<1, false>);
+    }
     return hipGetLastError();
 }
 

@@ -128,7 +128,7 @@ struct jev_ctx {
     int cap = 0, len = 0;
 
     // workspace
-    DevBuf<float> h, y, yo, ydown, q, x32, f32, xn, logits, part, xsum, cap32;
+    DevBuf<float> h, y, yo, ydown, q, x32, f32, xn, logits, part, apart, xsum, cap32;
     DevBuf<uint16_t> xt, ft; // fp16 pairs in the GEMM operand-tile layout
     DevBuf<int32_t> ints, dec_state;
     DevBuf<AttnTile> tiles;
@@ -501,6 +501,7 @@ struct Plan {
     const int32_t *d_tokens = nullptr, *d_slot = nullptr, *d_pos = nullptr, *d_slo = nullptr, *d_shi = nullptr,
                   *d_seg = nullptr, *d_out = nullptr, *d_rows = nullptr;
     int n_tiles = 0;
+    AttnSchedule attn; // how the tiles' attention is cut into workgroups
     // every attention tile a single token (rows of one token each): the
     // decode attention serves them, its chunks combined per token
     bool single_rows = false;
@@ -571,6 +572,7 @@ int build_plan(jev_ctx *c, const int32_t *tokens, bool tokens_on_device, int T, 
     std::vector<AttnTile> &tiles = c->host_tiles;
     tiles.clear();
     int max_limit = 0;
+    double key_blocks = 0; // 64-key blocks over all tiles
     for (int t = 0; t < T;) {
         auto at = [&](int i, int &slot, int &lo, int &hi, int &seg) {
             if (L) {
@@ -597,7 +599,9 @@ int build_plan(jev_ctx *c, const int32_t *tokens, bool tokens_on_device, int T, 
         AttnTile tile{t, n, lo0, hi0, seg0, s0, 0, 0};
         tiles.push_back(tile);
         for (int i = 0; i < n; i++) p.visible_pairs += (double)(hi0 - lo0) + (s0 + i - seg0 + 1);
-        max_limit = std::max(max_limit, (hi0 - lo0) + (s0 + n - 1 - seg0 + 1));
+        const int limit = (hi0 - lo0) + (s0 + n - 1 - seg0 + 1);
+        max_limit = std::max(max_limit, limit);
+        key_blocks += (limit + 63) / 64;
         t += n;
     }
     p.n_tiles = (int)tiles.size();
@@ -607,6 +611,8 @@ int build_plan(jev_ctx *c, const int32_t *tokens, bool tokens_on_device, int T, 
     // of how many rows run -- so a rows step takes the same attention kernel
     // whether it is replayed from a graph or run step by step
     p.single_rows = L && T >= 2 && p.n_tiles == T;
+    if (T >= 2 && !p.single_rows)
+        p.attn = attn_schedule(p.n_tiles, c->cfg.n_heads, c->cfg.n_heads / c->cfg.n_kv_heads, (max_limit + 63) / 64, key_blocks);
     if (p.single_rows) {
         std::vector<int32_t> fresh(L->slot, L->slot + T);
         std::sort(fresh.begin(), fresh.end());
@@ -990,6 +996,8 @@ int enqueue_forward(jev_ctx *c, const Plan &p, int mode, int n_rows, float *dout
             aa.cap = c->cap;
             aa.scale = scale;
             aa.ot = c->xt.p;
+            aa.sched = p.attn;
+            aa.part = c->apart.p;
             {
                 ProfScope ps(c, JEV_PROF_ATTN, 4.0 * f.head_dim * f.n_heads * p.visible_pairs,
                              8.0 * f.head_dim * f.n_kv_heads * p.kv_rows + 8.0 * T * qdim, true);
@@ -1218,6 +1226,7 @@ int prepare(jev_ctx *c, const int32_t *tokens, bool on_device, int T, const jev_
     if (rc) return rc;
     rc = build_plan(c, tokens, on_device, T, layout, mode, rows, n_rows, p);
     if (rc) return rc;
+    HIP_TRY(c->apart.ensure(p.attn.floats));
     return ensure_workspace(c, T, p.n_out, mode, p.max_chunks, p.single_rows);
 }
 
@@ -1306,7 +1315,7 @@ void jev_destroy(jev_ctx *c)
     if (c->vp) (void)hipFree(c->vp);
     c->h.release(); c->y.release(); c->yo.release(); c->ydown.release(); c->q.release();
     c->x32.release(); c->f32.release(); c->xn.release(); c->logits.release();
-    c->part.release(); c->xsum.release(); c->cap32.release(); c->xt.release(); c->ft.release(); c->ints.release(); c->dec_state.release(); c->tiles.release(); c->amax_v.release(); c->amax_i.release();
+    c->part.release(); c->apart.release(); c->xsum.release(); c->cap32.release(); c->xt.release(); c->ft.release(); c->ints.release(); c->dec_state.release(); c->tiles.release(); c->amax_v.release(); c->amax_i.release();
     if (c->pin_ints) (void)hipHostFree(c->pin_ints);
     if (c->pin_tiles) (void)hipHostFree(c->pin_tiles);
     if (c->pin_out) (void)hipHostFree(c->pin_out);
