@@ -115,6 +115,29 @@ __device__ __forceinline__ half8_t decode_b_frag(const BChunk &c, int bb)
 // NW: waves per workgroup, side by side along N (BN = 16 TN NW).  All of them
 // share one activation tile: the wider the workgroup, the fewer activation
 // loads and LDS stores per MFMA.
+// Tile pairs by which a tile's scale FMAs trail its MFMA pair (0: right after
+// it, where they wait for the matrix core unless other waves fill in), and
+// whether the scale is converted once instead of inside every FMA
+// (v_fma_mix_f32 takes the fp16 scale as it is but issues slower than a plain
+// FMA).  Both are settled per tile by timing, cold weights, 3B projections, us:
+//   4 x 2 and 4 x 4 tiles: two pairs; 4 x 2 with plain FMAs but for Q4_0 (Q5_1
+//     QKV 1500 rows 160 -> 149, down 236 -> 219, SwiGLU 640 193 -> 178; SwiGLU
+//     256 rows Q8_0 81 -> 72, Q5_1 100 -> 84)
+//   2 x 1: two pairs and plain FMAs (Q8_0 QKV 96 rows 14.9 -> 13.9, Q4_0 down
+//     20.6 -> 18.6)
+//   1 x 1, 1 x 2: one pair (Q8_0 down 32 rows 12.6 -> 11.8, Q5_1 16.3 -> 15.0)
+//   2 x 2: neither (two to four waves per SIMD fill in: 160 rows 16.9 -> 17.4
+//     with two pairs), except Q5_1 at four waves per SIMD, where they leave
+//     room in its 128 registers (SwiGLU 200 rows 97 -> 68)
+constexpr int bd_lag(int type, int tm, int tn, int nw)
+{
+    return tm * tn >= 8 || (tm == 2 && tn == 1) || (type == kQ5_1 && nw >= 14) ? 2 : tm == 1 ? 1 : 0;
+}
+constexpr bool bd_plain_scale(int type, int tm, int tn, int nw)
+{
+    return (tm == 2 && tn == 1) || (tm * tn == 8 && type != kQ4_0) || (type == kQ5_1 && nw >= 14);
+}
+
 template <int TYPE, int MODE, int TM, int TN, int PD, int OCC, bool FOLD = false, int NW = 4>
 __global__ __launch_bounds__(64 * NW, OCC) void gemm_bd_kernel(GemmArgs a, int mt, int nt, int gm)
 {
@@ -278,14 +301,11 @@ __global__ __launch_bounds__(64 * NW, OCC) void gemm_bd_kernel(GemmArgs a, int m
         }
     };
 
-    // Large tiles: the scale FMAs of a tile trail its MFMA pair by two pairs
-    // (the result is ready by then, so the vector ALU works beside the matrix
-    // core instead of waiting on it; 2-4 % at 4528 rows, nothing at 256).
-    // Each accumulator still takes its blocks' FMAs in block order, so the
-    // arithmetic is that of the plain order.
+    // Each accumulator takes its blocks' FMAs in block order whatever the lag
+    // is, so the arithmetic is that of the plain order.
     auto compute = [&](int st, int buf, const BChunk (&br)[TN]) __attribute__((always_inline)) {
         const bool second = 2 * st + 1 < nb;
-        constexpr int LAG = TM * TN >= 16 ? 2 : 0, NQ = 2 * TM * TN;
+        constexpr int LAG = bd_lag(TYPE, TM, TN, NW), NQ = 2 * TM * TN;
         floatx4 pq[LAG > 0 ? LAG : 1], xq[LAG > 0 ? LAG : 1];
         float dq[LAG > 0 ? LAG : 1], mq[LAG > 0 ? LAG : 1];
         auto apply = [&](int t) __attribute__((always_inline)) {
@@ -311,6 +331,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void gemm_bd_kernel(GemmArgs a, int m
                 dv[n] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, h2f((uint16_t)(bb ? br[n].d >> 16 : br[n].d))) & live);
                 if (TYPE == kQ5_1)
                     mv[n] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, h2f((uint16_t)(bb ? br[n].m >> 16 : br[n].m))) & live);
+                if constexpr (bd_plain_scale(TYPE, TM, TN, NW)) {
+                    asm("" : "+v"(dv[n])); // not foldable into the FMAs
+                    if (TYPE == kQ5_1) asm("" : "+v"(mv[n]));
+                }
             }
 #pragma unroll
             for (int mi = 0; mi < TM; mi++) {
@@ -776,12 +800,14 @@ static hipError_t launch_mode(const GemmArgs &a, hipStream_t s)
     // per weight row group, 1.5-2x the B-direct kernel there (12 rows of the
     // Q5_1 3B shape: 2.1 against 3.6 ms of GEMM per step)
     if (a.M <= 16) return launch_skinny<TYPE, MODE, 4, 8>(a, s);
-    int tcols; // 16-wide tile columns of the output (gate and up both count)
+    int tcols;           // 16-wide tile columns of the output (gate and up both count)
+    bool one_seg = true; // a four-wave tile of 128 or 256 columns lies in one segment
     if (MODE == kGemmSwiGlu) {
         tcols = 2 * (a.seg[0].rows / 16);
     } else {
         int ntot = 0;
         for (int i = 0; i < a.nseg; i++) ntot += a.seg[i].rows;
+        for (int i = 0; i + 1 < a.nseg; i++) one_seg = one_seg && a.seg[i].rows % 256 == 0;
         tcols = (ntot + 15) / 16;
     }
     // workgroups of a grid of 16 tm x 16 tn nw tiles
@@ -794,11 +820,8 @@ static hipError_t launch_mode(const GemmArgs &a, hipStream_t s)
             if (wgs(2, 2, 8) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 8>(a, s, 4);
             if (wgs(2, 2, 10) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 10>(a, s, 4);
             if (wgs(2, 2, 12) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 12>(a, s, 4);
-            if constexpr (TYPE != kQ5_1) {
-                // (four waves per SIMD leave 128 registers: Q5_1's block sums do not fit, 74 -> 98 us at 192 rows)
-                if (wgs(2, 2, 14) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 14>(a, s, 4);
-                if (wgs(2, 2, 16) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 16>(a, s, 4);
-            }
+            if (wgs(2, 2, 14) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 14>(a, s, 4);
+            if (wgs(2, 2, 16) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 16>(a, s, 4);
             // 64-row tiles (half the decode per MFMA) where their grid nearly
             // fills the round; nine waves only when the last tile is more than
             // half full (208 rows of Q5_1: 76 -> 86 us)
@@ -819,16 +842,19 @@ static hipError_t launch_mode(const GemmArgs &a, hipStream_t s)
         if (wgs(2, 1, 12) <= kCUs) return launch_bd<TYPE, MODE, 2, 1, 1, 1, false, 12>(a, s);
         if (wgs(2, 2, 8) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 8>(a, s);
         if (wgs(2, 2, 12) <= kCUs) return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 12>(a, s);
-        // two or three per CU; Q5_1's second FMA per output favours the taller tile (512 rows of QKV 68.3 -> 55.9 us)
+        // two or three per CU, eight waves of 32 rows (Q5_1, whose second FMA per
+        // output favours fewer columns: 64 rows of half the width) unless
+        // four-wave workgroups leave the busiest CU fewer waves (400 rows of
+        // Q4_0 QKV 43.6 -> 41.1 us; equal counts go to the wider one, 457
+        // rows 47.3 -> 44.7)
+        const long wide = TYPE == kQ5_1 ? wgs(4, 1, 8) : wgs(2, 2, 8);
+        if ((wgs(2, 2, 4) + kCUs - 1) / kCUs < 2 * ((wide + kCUs - 1) / kCUs)) return launch_bd<TYPE, MODE, 2, 2, 1, 4, false, 4>(a, s);
         if constexpr (TYPE == kQ5_1) return launch_bd<TYPE, MODE, 4, 1, 1, 1, false, 8>(a, s);
         return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 8>(a, s);
     }
     // Large batches.  Four-wave 64 x 256 tiles keep 16 tiles per wave, and
     // with them Q5_1 has no registers for its byte quants: eight waves of 64 x
-    // 32 there at every size.  A four-wave tile must lie in one segment.
-    bool one_seg = true;
-    if (MODE == kGemmStore)
-        for (int i = 0; i + 1 < a.nseg; i++) one_seg = one_seg && a.seg[i].rows % 256 == 0;
+    // 32 there at every size.
     if constexpr (MODE == kGemmStore && TYPE != kQ5_1)
         if (a.fold) return launch_bd<TYPE, MODE, 4, 4, 1, 2, true>(a, s);
     if (TYPE == kQ5_1 || !one_seg || (MODE == kGemmStore && wgs(4, 2, 8) <= 2 * kCUs))
