@@ -118,6 +118,30 @@ __device__ __forceinline__ void bytes_to_f16(uint32_t bytes, _Float16 bias, uint
     p23 = sub_bias(biased_pair(bytes, 0x04030402u), bias);
 }
 
+// Bit i of a 4-bit value x << 4 to bit 8 i + 4 (masked by the caller):
+// (x << 4) * 0x204081 (both fit 24 bits) on the full-rate 24-bit multiplier
+// (the compiler picks the quarter-rate 32-bit one for the plain product).
+__device__ __forceinline__ uint32_t spread4(uint32_t x)
+{
+    uint32_t r;
+    asm("v_mul_u32_u24 %0, %1, %2" : "=v"(r) : "v"(x), "v"(0x00204081u));
+    return r;
+}
+
+// A block's B fragment from Q5_1's fields: `nib` the lane's four bytes of
+// nibbles, the low byte of `qh` its fifth bits; exact integers in [0, 31].
+__device__ __forceinline__ half8_t decode_q5_frag(uint32_t nib, uint32_t qh)
+{
+    uint32_t n0 = nib & 0x0f0f0f0fu, n1 = (nib >> 4) & 0x0f0f0f0fu;
+    const uint32_t hb = qh & 0xffu;
+    n0 |= spread4((hb & 15u) << 4) & 0x10101010u;
+    n1 |= spread4(hb & 0xf0u) & 0x10101010u;
+    uint32_t o0, o1, o2, o3;
+    bytes_to_f16(n0, (_Float16)1024.0f, o0, o1);
+    bytes_to_f16(n1, (_Float16)1024.0f, o2, o3);
+    return __builtin_bit_cast(half8_t, make_uint4(o0, o1, o2, o3));
+}
+
 __device__ __forceinline__ float warp_sum(float v)
 {
 #pragma unroll

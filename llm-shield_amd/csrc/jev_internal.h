@@ -38,8 +38,9 @@ int64_t row_bytes(int type, int64_t cols);
 //                          Q8_0's order (lane l's 16 bytes at 16 l), for the
 //                          kernels of two or more tokens: one byte permute and
 //                          one packed subtraction per two weights instead of the
-//                          nibble and fifth-bit assembly (the one-token GEMV keeps
-//                          the 5-bit fields, whose bytes it streams)
+//                          nibble and fifth-bit assembly (the one-token GEMV and the
+//                          few-row vocabulary head keep the 5-bit fields, whose
+//                          bytes they stream)
 constexpr int kTileRows = 16, kTileK = 64;
 struct QWeight {
     int type = -1;

@@ -45,6 +45,8 @@ namespace jev {
 
 namespace {
 
+constexpr int kCUs = 256;
+
 // One loader chunk: a lane slot of a weight tile -- the quants of one row
 // at k = 8g .. 8g + 7 of both blocks of the stage -- and that row's scales.
 struct BChunk {
@@ -498,27 +500,49 @@ __global__ __launch_bounds__(64 * NW, OCC) void gemm_bd_kernel(GemmArgs a, int m
 // Skinny variant for M <= 16 (one row group: the reasoning decider's rows,
 // short branches).  The B-direct grid at such M is N / 128 x splits
 // workgroups -- 96 for a 3072-row projection split 4 -- and leaves most of the
-// chip's load bandwidth idle.  Here each wave owns one 16-row weight group
-// (SwiGLU: the gate and the up group of the same outputs) and the workgroup's
-// four waves one K split, 8x the waves of B-direct.  Each wave streams its
-// weights through its own U-stage register ring; the activation fragments
-// (and Q5_1 block sums), the same for all four waves, are staged into LDS
-// once per workgroup in chunks of CH stages, double buffered, with one
-// barrier per chunk: loaded into registers at the top of the chunk before,
-// written to LDS at its end.  (Direct-to-LDS loads would save the registers,
-// but the compiler then drains every outstanding load before the first LDS
-// read after them, the weight ring included, once per chunk.)  Per output it issues exactly
-// gemm_bd_kernel's sequence: per block p = mfma(x_hi, q); p = mfma(x_lo, q,
-// p); acc = fma(d, p, acc) (+ fma(m, sum x, acc)), blocks ascending within the
-// split, the same clamped operands for an odd last block -- so its results
-// are the same bits.
-template <int TYPE, int MODE, int U, int CH>
-__global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(GemmArgs a, int ngroups, int nq)
+// chip's load bandwidth idle.  Here each wave owns TN 16-row weight groups over
+// one K split and streams them through its own register ring of CH stages,
+// while the activation fragments (and Q5_1 block sums), the same for all waves
+// of the workgroup, go through LDS in chunks of CH stages, double buffered,
+// one barrier per chunk.
+//
+// Bound by the chain of one wave's stages (the 3B projections give 0.75 waves
+// per SIMD) and, for the vocabulary head, by the weight bytes.  So:
+//  * A ring slot holds a stage's weights and this wave's share of the
+//    activations CH stages further on, loaded and retired together.  Loads
+//    retire in order, so nothing ever waits for a load younger than its own
+//    stage; with the activations loaded once per chunk, the wait for them at
+//    the chunk's end also drained the weight ring.
+//  * Loads stay at the end of their stage (the sched_barriers): left alone, the
+//    compiler sinks them to their use.
+//  * LDS reads run one block ahead; for one Q5_1 group per wave the scale FMAs
+//    trail their MFMA pair by one block with the scales converted once.  (The
+//    other types issue too few vector instructions for that to hide the pair.)
+//  * SwiGLU: gate and up in neighbouring waves (GU), twice the waves, the
+//    up sums handed over through LDS at the end.
+//  * One round of at most 256 workgroups, each as wide as that needs
+//    (launch_skinny), since a CU with a second workgroup finishes last.
+// 12 rows, cold weights, 3B projections, us, before -> now: Q5_1 QKV 9.3 ->
+// 8.3, O 7.4 -> 6.6, gate/up 21.7 -> 19.7, down 12.3 -> 10.4, head 97 -> 72;
+// Q8_0 QKV 7.8 -> 6.8, gate/up 19.1 -> 16.0, down 10.0 -> 8.2, head 88 -> 76;
+// Q4_0 gate/up 17.1 -> 13.0, head 73 -> 49.
+//
+// Per output it issues exactly gemm_bd_kernel's sequence: per block p =
+// mfma(x_hi, q); p = mfma(x_lo, q, p); acc = fma(d, p, acc) (+ fma(m, sum x,
+// acc)), blocks ascending within the split -- so its results are the same bits.
+// The missing second block of an odd K reads a finite neighbour's activations
+// against the layout's zero scales.
+// F5: Q5_1 quants from the 5-bit fields (two thirds of the byte copy's bytes,
+// more decode) instead of the byte copy.
+template <int TYPE, int MODE, int TN, int NW, bool F5>
+__global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(GemmArgs a, int ngroups, int nq)
 {
-    constexpr int TN = MODE == kGemmSwiGlu ? 2 : 1;
-    constexpr int NB = 2 * TN; // weight loads per stage
-    static_assert(CH % U == 0, "ring slots restart at every chunk");
-    static_assert(CH * NB + CH + 1 <= 63, "outstanding loads beyond the vmcnt range");
+    constexpr bool GU = MODE == kGemmSwiGlu;
+    constexpr int CH = 4;                                    // stages per chunk and ring turn
+    constexpr int LAG = TYPE == kQ5_1 && TN == 1 ? 1 : 0;    // blocks the scale FMAs trail
+    constexpr int GW = GU ? NW / 2 : NW * TN;                // row groups per workgroup
+    static_assert(!GU || (TN == 1 && NW % 2 == 0), "gate and up in neighbouring waves");
+    static_assert(CH * 32 <= 64 * NW, "one block sum per thread");
     __shared__ __attribute__((aligned(16))) uint4 As[2][CH * 4 * 64]; // [stage][block][part][lane]
     __shared__ __attribute__((aligned(16))) float Xs[2][TYPE == kQ5_1 ? CH * 2 * 16 : 4]; // [block][row]
 
@@ -528,30 +552,28 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(GemmArgs a, int ngr
     // vector ALU with the decode and the scale FMAs.
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int z = __builtin_amdgcn_readfirstlane((int)blockIdx.x / nq), q = blockIdx.x - z * nq;
-    const int g = q * 4 + wave;              // this wave's row group; past ngroups: loads only
-    const int gl = min(g, ngroups - 1);
+    const int g0 = q * GW + (GU ? wave >> 1 : wave * TN);    // this wave's first row group; past ngroups: loads only
     const int M = a.M, K = a.K, nblk = K >> 5;
     const int nb_per = __builtin_amdgcn_readfirstlane(gemm_split_blocks(nblk, a.ksplit));
     const int kb_begin = z * nb_per;
     const int nb = min(nblk - kb_begin, nb_per);
-    const int nstage = (nb + 1) >> 1;
-    const int nchunk = __builtin_amdgcn_readfirstlane((nstage + CH - 1) / CH);
+    const int nstage = __builtin_amdgcn_readfirstlane((nb + 1) >> 1);
 
     const rsrc_t ra = make_rsrc(a.xt, (uint32_t)nblk * 2048); // row group 0 of the operand tiles
     rsrc_t rs;
     if (TYPE == kQ5_1) rs = make_rsrc(a.xsum, (uint32_t)M * nblk * 4);
 
-    // weights: tile n of this wave
-    constexpr bool BQ = kByteQuants<TYPE>;
-    rsrc_t rq[TN], rd[TN];
+    // weights: group n of this wave
+    constexpr bool BQ = kByteQuants<TYPE> && !F5;
+    rsrc_t rq[TN], rd[TN], rh[TN];
     int btile0[TN];
-    int seg_store = 0, start_store = 0;
-    const uint32_t vq = (uint32_t)lane * (BQ ? 16 : 8), vd = 4 * (lane & 15);
+    const uint32_t vq = (uint32_t)lane * (BQ ? 16 : 8), vd = 4 * (lane & 15), vh = 2 * lane;
 #pragma unroll
     for (int n = 0; n < TN; n++) {
+        const int gl = min(g0 + n, ngroups - 1);
         int seg, rgw;
-        if (MODE == kGemmSwiGlu) {
-            seg = n;
+        if (GU) {
+            seg = wave & 1;
             rgw = gl;
         } else {
             int s0 = 0, start = 0;
@@ -561,53 +583,35 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(GemmArgs a, int ngr
             }
             seg = s0;
             rgw = (gl * 16 - start) / 16;
-            seg_store = s0;
-            start_store = start;
         }
         seg = __builtin_amdgcn_readfirstlane(seg);
         const QWeight &wt = a.seg[seg];
         const int KP = tile_kpairs(wt.cols), RG = tile_rows(wt.rows);
         const uint32_t tiles = (uint32_t)RG * KP;
-        rq[n] = quant_rsrc<TYPE>(wt, tiles);
+        rq[n] = F5 ? make_rsrc(wt.qs, tiles * 512u) : quant_rsrc<TYPE>(wt, tiles);
         rd[n] = make_rsrc(wt.d, tiles * tile_d_bytes(TYPE));
+        if (F5) rh[n] = make_rsrc(wt.qh, tiles * 128u);
         btile0[n] = __builtin_amdgcn_readfirstlane(min(rgw, RG - 1) * KP + (kb_begin >> 1));
     }
-    auto load_b = [&](int st, BChunk (&br)[TN]) __attribute__((always_inline)) {
+
+    // Activation fragment f = block * 2 + part of a stage, one KiB each: wave f
+    // takes it (waves past the fourth repeat the last: the same bytes to the
+    // same slot); eight waves take half a fragment each.
+    auto load_a = [&](int st) __attribute__((always_inline)) -> uint4 {
         st = min(st, nstage - 1);
-#pragma unroll
-        for (int n = 0; n < TN; n++) {
-            const int tile = __builtin_amdgcn_readfirstlane(btile0[n] + st);
-            if (BQ) {
-                br[n].q = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rq[n], vq, tile * 1024, 0));
-            } else {
-                uint2 v = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rq[n], vq, tile * 512, 0));
-                br[n].q = make_uint4(v.x, v.y, 0u, 0u);
-            }
-            if (TYPE == kQ5_1) {
-                const uint2 dm = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rd[n], 2 * vd, tile * 128, 0));
-                br[n].d = dm.x;
-                br[n].m = dm.y;
-            } else {
-                br[n].d = __builtin_amdgcn_raw_buffer_load_b32(rd[n], vd, tile * 64, 0);
-            }
-        }
+        const int f = NW == 8 ? wave >> 1 : min(wave, 3);
+        const int kblk = kb_begin + min(2 * st + (f >> 1), nb - 1);
+        // the offset is wave-uniform; as a vector value it would cost a one-pass loop per load
+        const int soff = __builtin_amdgcn_readfirstlane((kblk * 2 + (f & 1)) * 1024);
+        if (NW != 8) return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, lane * 16, soff, 0));
+        const uint2 v = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(ra, (wave & 1) * 512 + lane * 8, soff, 0));
+        return make_uint4(v.x, v.y, 0u, 0u);
     };
-    // Chunk c's activation fragments: this wave's CH of the chunk's 4 * CH,
-    // fragment f = stage * 4 + block * 2 + part, one KiB each.
-    auto load_a = [&](int c, uint4 (&ar)[CH]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < CH; i++) {
-            const int f = wave * CH + i;
-            const int st = min(c * CH + (f >> 2), nstage - 1);
-            const int kblk = kb_begin + min(2 * st + ((f >> 1) & 1), nb - 1);
-            // the offset is wave-uniform; as a vector value it would cost a one-pass loop per load
-            const int soff = __builtin_amdgcn_readfirstlane((kblk * 2 + (f & 1)) * 1024);
-            ar[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, lane * 16, soff, 0));
-        }
-    };
-    auto store_a = [&](int buf, const uint4 (&ar)[CH]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < CH; i++) As[buf][(wave * CH + i) * 64 + lane] = ar[i];
+    auto store_a = [&](int buf, int j, const uint4 &v) __attribute__((always_inline)) {
+        if (NW != 8)
+            As[buf][(j * 4 + min(wave, 3)) * 64 + lane] = v;
+        else
+            ((uint2 *)&As[buf][(j * 4 + (wave >> 1)) * 64])[(wave & 1) * 64 + lane] = make_uint2(v.x, v.y);
     };
     // Chunk c's block sums, thread t: block t / 16 of the chunk, row t % 16
     // (the address gemm_bd_kernel reads for that row and block).
@@ -621,132 +625,255 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_kernel(GemmArgs a, int ngr
         const uint32_t off = ((uint32_t)(e & 15) * nblk + kb_begin + 2 * st + (bl & 1)) * 4;
         return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
     };
+    auto store_xs = [&](int buf, float v) __attribute__((always_inline)) {
+        if (TYPE == kQ5_1 && tid < CH * 32) Xs[buf][tid] = v;
+    };
+    struct Slot {
+        BChunk b[TN];
+        uint32_t qh[TN];
+        uint4 a;  // of stage st + CH
+        float xs; // of the next chunk, in a chunk's first slot
+    };
+    // Slot of stage s0 + j (s0 a chunk's first stage).  Past the last stage
+    // everything repeats it, into slots and buffers nobody reads, so every
+    // chunk issues the same loads and the compiler's wait counts hold.
+    auto load = [&](int s0, int j, Slot &s) __attribute__((always_inline)) {
+        const int st = min(s0 + j, nstage - 1);
+#pragma unroll
+        for (int n = 0; n < TN; n++) {
+            const int tile = __builtin_amdgcn_readfirstlane(btile0[n] + st);
+            if (BQ) {
+                s.b[n].q = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rq[n], vq, tile * 1024, 0));
+            } else {
+                uint2 v = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rq[n], vq, tile * 512, 0));
+                s.b[n].q = make_uint4(v.x, v.y, 0u, 0u);
+            }
+            if (TYPE == kQ5_1) {
+                const uint2 dm = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rd[n], 2 * vd, tile * 128, 0));
+                s.b[n].d = dm.x;
+                s.b[n].m = dm.y;
+                if (F5) s.qh[n] = __builtin_amdgcn_raw_buffer_load_b16(rh[n], vh, tile * 128, 0);
+            } else {
+                s.b[n].d = __builtin_amdgcn_raw_buffer_load_b32(rd[n], vd, tile * 64, 0);
+            }
+        }
+        s.a = load_a(s0 + j + CH);
+        if (TYPE == kQ5_1 && j == 0) s.xs = load_xs(s0 / CH + 1);
+    };
 
     floatx4 acc[TN];
 #pragma unroll
     for (int n = 0; n < TN; n++) acc[n] = floatx4{0.f, 0.f, 0.f, 0.f};
-    auto compute = [&](int st, int buf, int sl, const BChunk (&br)[TN]) __attribute__((always_inline)) {
-        const bool second = 2 * st + 1 < nb;
+    struct Frag {
+        half8_t ah, al;
+        floatx4 xs; // block sums of the lane's four C rows
+    };
+    struct Pair { // a block's unscaled products and what scales them
+        floatx4 p, xs;
+        float d, m;
+    };
+    auto read = [&](int buf, int i, Frag &f) __attribute__((always_inline)) {
+        f.ah = __builtin_bit_cast(half8_t, As[buf][(i * 2 + 0) * 64 + lane]);
+        f.al = __builtin_bit_cast(half8_t, As[buf][(i * 2 + 1) * 64 + lane]);
+        if (TYPE == kQ5_1) f.xs = *(const floatx4 *)&Xs[buf][i * 16 + 4 * (lane >> 4)];
+    };
+    auto apply = [&](int n, const Pair &t) __attribute__((always_inline)) {
 #pragma unroll
-        for (int bb = 0; bb < 2; bb++) {
-            const uint32_t live = bb == 0 || second ? ~0u : 0u;
-            const half8_t ah = __builtin_bit_cast(half8_t, As[buf][(sl * 4 + bb * 2 + 0) * 64 + lane]);
-            const half8_t al = __builtin_bit_cast(half8_t, As[buf][(sl * 4 + bb * 2 + 1) * 64 + lane]);
-            floatx4 xs4;
-            if (TYPE == kQ5_1) xs4 = *(const floatx4 *)&Xs[buf][(sl * 2 + bb) * 16 + 4 * (lane >> 4)];
+        for (int r = 0; r < 4; r++) {
+            float v = fmaf(t.d, t.p[r], acc[n][r]);
+            if (TYPE == kQ5_1) v = fmaf(t.m, t.xs[r], v);
+            acc[n][r] = v;
+        }
+    };
+    Pair late;
+    // block bb of the slot's stage; first: nothing trails it yet
+    auto block = [&](const Frag &f, const Slot &s, int bb, bool first) __attribute__((always_inline)) {
 #pragma unroll
-            for (int n = 0; n < TN; n++) {
-                const half8_t bf = decode_b_frag<TYPE>(br[n], bb);
-                const float dv = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, h2f((uint16_t)(bb ? br[n].d >> 16 : br[n].d))) & live);
-                float mv = 0.f;
-                if (TYPE == kQ5_1)
-                    mv = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, h2f((uint16_t)(bb ? br[n].m >> 16 : br[n].m))) & live);
-                floatx4 p = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bf, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                p = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bf, p, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    float v = fmaf(dv, p[r], acc[n][r]);
-                    if (TYPE == kQ5_1) v = fmaf(mv, xs4[r], v);
-                    acc[n][r] = v;
-                }
+        for (int n = 0; n < TN; n++) {
+            half8_t bf;
+            if constexpr (F5)
+                bf = decode_q5_frag(bb ? s.b[n].q.y : s.b[n].q.x, s.qh[n] >> (8 * bb));
+            else
+                bf = decode_b_frag<TYPE>(s.b[n], bb);
+            Pair t;
+            t.d = h2f((uint16_t)(bb ? s.b[n].d >> 16 : s.b[n].d));
+            if (TYPE == kQ5_1) {
+                t.m = h2f((uint16_t)(bb ? s.b[n].m >> 16 : s.b[n].m));
+                t.xs = f.xs;
+            }
+            if constexpr (LAG > 0) {
+                asm("" : "+v"(t.d)); // not foldable into the FMAs
+                asm("" : "+v"(t.m));
+            }
+            t.p = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.ah, bf, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            t.p = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.al, bf, t.p, 0, 0, 0);
+            if constexpr (LAG > 0) {
+                if (!first) apply(n, late);
+                late = t;
+            } else {
+                apply(n, t);
             }
         }
     };
 
-    // ---- pipeline.  Issue order per chunk c: the activations and block sums
-    // of chunk c + 1 (registers, written to the other LDS buffer at the end of
-    // chunk c), then one weight stage per stage of chunk c, U stages ahead.
-    BChunk br[U][TN];
-    uint4 ar[CH];
-    float xr = load_xs(0);
-    load_a(0, ar);
+    // ---- pipeline
+    Slot ring[CH];
+    {
+        uint4 a0[CH];
+        const float x0 = load_xs(0);
 #pragma unroll
-    for (int t = 0; t < U; t++) load_b(t, br[t]);
-    store_a(0, ar);
-    if (TYPE == kQ5_1 && tid < CH * 32) Xs[0][tid] = xr;
-    // Unconditional, so every chunk issues the same loads (the last one
-    // re-reads clamped stages into a buffer nobody reads): with a branch
-    // around them the compiler's wait counts at the chunk top assume the
-    // shorter path and wait on the activation loads just issued.
-    for (int c = 0; c < nchunk; c++) {
-        const int buf = c & 1;
-        __syncthreads(); // chunk c staged by everyone; chunk c - 1's buffers are free
-        xr = load_xs(c + 1);
-        load_a(c + 1, ar);
+        for (int j = 0; j < CH; j++) a0[j] = load_a(j);
 #pragma unroll
         for (int j = 0; j < CH; j++) {
-            const int st = c * CH + j;
-            if (st < nstage) compute(st, buf, j, br[j % U]);
-            load_b(st + U, br[j % U]);
+            load(0, j, ring[j]);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        store_a(buf ^ 1, ar);
-        if (TYPE == kQ5_1 && tid < CH * 32) Xs[buf ^ 1][tid] = xr;
+#pragma unroll
+        for (int j = 0; j < CH; j++) store_a(0, j, a0[j]);
+        store_xs(0, x0);
+    }
+    const int nfull = nstage / CH;
+    for (int c = 0; c < nfull; c++) {
+        const int buf = c & 1;
+        __syncthreads(); // chunk c staged by everyone; chunk c - 1's buffer is free
+        __builtin_amdgcn_sched_barrier(0);
+        Frag fr[2];
+        read(buf, 0, fr[0]);
+#pragma unroll
+        for (int j = 0; j < CH; j++) {
+#pragma unroll
+            for (int bb = 0; bb < 2; bb++) {
+                const int i = 2 * j + bb;
+                if (i + 1 < 2 * CH) read(buf, i + 1, fr[(i + 1) & 1]);
+                block(fr[i & 1], ring[j], bb, i == 0);
+            }
+            store_a(buf ^ 1, j, ring[j].a);
+            if (j == 0) store_xs(buf ^ 1, ring[j].xs);
+            load((c + 1) * CH, j, ring[j]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (LAG > 0) apply(0, late);
+    }
+    {
+        const int rem = nstage - nfull * CH, buf = nfull & 1; // the last stages
+        if (rem > 0) {
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < CH - 1; j++) {
+                if (j < rem) {
+                    Frag f0, f1;
+                    read(buf, 2 * j, f0);
+                    read(buf, 2 * j + 1, f1);
+                    block(f0, ring[j], 0, true);
+                    block(f1, ring[j], 1, false);
+                    if constexpr (LAG > 0) apply(0, late);
+                }
+            }
+        }
     }
 
     // ---- epilogue.  Lane holds C[4*(lane/16) + r][lane % 16].
     const int row_base = 4 * (lane >> 4);
     if (MODE == kGemmStore) {
-        if (g >= ngroups) return;
-        const QWeight &ws = a.seg[seg_store];
-        if (g * 16 - start_store + (lane & 15) >= ws.rows) return;
-        float *y = a.y + (size_t)z * M * a.ldy + g * 16 + (lane & 15);
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-            if (row_base + r < M) __builtin_nontemporal_store(acc[0][r], &y[(size_t)(row_base + r) * a.ldy]);
-    } else {
-        const int ld = a.seg[0].rows;
-        const int col = g * 16 + (lane & 15);
-        const bool live = g < ngroups && col < ld;
-        __shared__ float es[16 * 64]; // [row][column of the workgroup's 64]: hi + lo of each output
+        for (int n = 0; n < TN; n++) {
+            // columns are the segments' rows concatenated; only the last
+            // segment may end inside a group
+            const int col = (g0 + n) * 16 + (lane & 15);
+            int end = 0;
+            for (int i = 0; i < a.nseg; i++) end += a.seg[i].rows;
+            if (col >= end) continue;
+            float *y = a.y + (size_t)z * M * a.ldy + col;
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int row = row_base + r;
-            // Kernels.SwiGlu (Kernels.cs:82-89): (g*u) * sigmoid(g).
-            const float gv = acc[0][r], u = acc[1][r];
-            const float gu = gv * u;
-            const float e = expf(-gv);
-            const float sg = 1.0f / (1.0f + e);
-            const float v = sg * gu;
-            uint16_t hi, lo;
-            split_f16(v, hi, lo);
-            if (live && row < M) {
-                a.ot[xt_index(row, col, ld >> 5, 0)] = hi;
-                a.ot[xt_index(row, col, ld >> 5, 1)] = lo;
-            }
-            if (a.osum) es[row * 64 + wave * 16 + (lane & 15)] = h2f(hi) + h2f(lo);
+            for (int r = 0; r < 4; r++)
+                if (row_base + r < M) __builtin_nontemporal_store(acc[n][r], &y[(size_t)(row_base + r) * a.ldy]);
         }
-        if (a.osum) {
-            // the Q5_1 block sums of these outputs for the down projection: the
-            // workgroup's four row groups are 64 consecutive columns, two whole
-            // blocks (ld is a multiple of 32), each summed in ascending column
-            // order as the block-sum kernel sums an operand tile
+    } else {
+        constexpr int NG = NW / 2; // row groups of the workgroup
+        const int ld = a.seg[0].rows;
+        floatx4 *up = (floatx4 *)&As[0][0];   // [group][lane]
+        float *es = (float *)&As[1][0];       // [row][column of the workgroup's]: hi + lo of each output
+        static_assert(NG * 64 <= CH * 4 * 64 && 16 * NG * 16 <= CH * 4 * 64 * 4, "the exchange fits the staging buffers");
+        __syncthreads(); // everyone is done with the staging buffers
+        if (wave & 1) up[(wave >> 1) * 64 + lane] = acc[0];
+        __syncthreads();
+        if (!(wave & 1)) {
+            const floatx4 u4 = up[(wave >> 1) * 64 + lane];
+            const int col = g0 * 16 + (lane & 15);
+            const bool live = g0 < ngroups && col < ld;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int row = row_base + r;
+                // Kernels.SwiGlu (Kernels.cs:82-89): (g*u) * sigmoid(g).
+                const float gv = acc[0][r], u = u4[r];
+                const float gu = gv * u;
+                const float e = expf(-gv);
+                const float sg = 1.0f / (1.0f + e);
+                const float v = sg * gu;
+                uint16_t hi, lo;
+                split_f16(v, hi, lo);
+                if (live && row < M) {
+                    a.ot[xt_index(row, col, ld >> 5, 0)] = hi;
+                    a.ot[xt_index(row, col, ld >> 5, 1)] = lo;
+                }
+                if (a.osum) es[row * 16 * NG + (wave >> 1) * 16 + (lane & 15)] = h2f(hi) + h2f(lo);
+            }
+        }
+        if (NG % 2 == 0 && a.osum) {
+            // the Q5_1 block sums of these outputs for the down projection: an
+            // even number of row groups is whole blocks of consecutive columns
+            // (ld is a multiple of 32), each summed in ascending column order
+            // as the block-sum kernel sums an operand tile
             __syncthreads();
-            const int row = tid & 15, blk = tid >> 4, c0 = q * 64 + 32 * blk;
-            if (tid < 32 && row < M && c0 < ld) {
+            const int row = tid & 15, blk = tid >> 4, c0 = q * 16 * NG + 32 * blk;
+            if (tid < 8 * NG && row < M && c0 < ld) {
                 float sum = 0.f;
-                for (int j = 0; j < 32; j++) sum += es[row * 64 + 32 * blk + j];
+                for (int j = 0; j < 32; j++) sum += es[row * 16 * NG + 32 * blk + j];
                 a.osum[(size_t)row * (ld >> 5) + (c0 >> 5)] = sum;
             }
         }
     }
 }
 
-template <int TYPE, int MODE, int U, int CH>
+template <int TYPE, int MODE, int TN, int NW, bool F5 = false>
+static hipError_t launch_skinny_cfg(const GemmArgs &a, int ngroups, hipStream_t s)
+{
+    constexpr int GW = MODE == kGemmSwiGlu ? NW / 2 : NW * TN;
+    const int nq = (ngroups + GW - 1) / GW;
+    launch_stamped(a.ev_start, a.ev_stop, gemm_skinny_kernel<TYPE, MODE, TN, NW, F5>, dim3(nq * a.ksplit), dim3(64 * NW), 0,
+                   s, a, ngroups, nq);
+    return hipGetLastError();
+}
+
+// As many waves per workgroup as one round of workgroups needs (12 rows, us,
+// 4 / 6 / 8 waves): Q8_0 store 16384 columns 12.8 / 14.1 / 16.4, 24576 20.5 /
+// 16.5 / 17.4, 32768 23.4 / 27.0 / 21.4; SwiGLU of 4096 outputs 10.0 / 12.1 /
+// 12.3, of 9216 19.2 / 16.0 / 18.2 (with the block sums, which take whole
+// blocks of columns, four or eight).  Past eight waves' one round, two groups
+// per wave share their activation reads (40960 columns: 28.4, one group 31.3
+// at best); from a full round of those on, Q5_1 is short of bytes rather than
+// of vector issue and reads the 5-bit fields (65536 columns 37.9 against 42.4
+// for the byte copy, 49152 39.0 against 34.4).
+template <int TYPE, int MODE>
 static hipError_t launch_skinny(const GemmArgs &a, hipStream_t s)
 {
-    int ngroups;
     if (MODE == kGemmSwiGlu) {
-        ngroups = a.seg[0].rows / 16;
-    } else {
-        // every segment but the last is a whole number of 16-row groups
-        int ntot = 0;
-        for (int i = 0; i < a.nseg; i++) ntot += a.seg[i].rows;
-        ngroups = (ntot + 15) / 16;
+        const int ngroups = a.seg[0].rows / 16;
+        if (ngroups <= 2 * kCUs) return launch_skinny_cfg<TYPE, MODE, 1, 4>(a, ngroups, s);
+        if (ngroups <= 3 * kCUs && !a.osum) return launch_skinny_cfg<TYPE, MODE, 1, 6>(a, ngroups, s);
+        return launch_skinny_cfg<TYPE, MODE, 1, 8>(a, ngroups, s);
     }
-    const int nq = (ngroups + 3) / 4;
-    launch_stamped(a.ev_start, a.ev_stop, gemm_skinny_kernel<TYPE, MODE, U, CH>, dim3(nq * a.ksplit), dim3(256), 0, s, a,
-                   ngroups, nq);
-    return hipGetLastError();
+    // every segment but the last is a whole number of 16-row groups
+    int ntot = 0;
+    for (int i = 0; i < a.nseg; i++) ntot += a.seg[i].rows;
+    const int ngroups = (ntot + 15) / 16;
+    auto fits = [&](int gw) { return (ngroups + gw - 1) / gw * a.ksplit <= kCUs; };
+    if (fits(4)) return launch_skinny_cfg<TYPE, kGemmStore, 1, 4>(a, ngroups, s);
+    if (fits(6)) return launch_skinny_cfg<TYPE, kGemmStore, 1, 6>(a, ngroups, s);
+    if (fits(8)) return launch_skinny_cfg<TYPE, kGemmStore, 1, 8>(a, ngroups, s);
+    if constexpr (TYPE == kQ5_1)
+        if ((ngroups + 15) / 16 * a.ksplit >= kCUs) return launch_skinny_cfg<TYPE, kGemmStore, 2, 8, true>(a, ngroups, s);
+    return launch_skinny_cfg<TYPE, kGemmStore, 2, 8>(a, ngroups, s);
 }
 
 // gm_cap: M tiles per group of the tile order (the tiles of a group that share
@@ -791,7 +918,6 @@ static hipError_t launch_bd(const GemmArgs &a, hipStream_t s, int gm_cap = 8)
 //   Q8_0 SwiGLU  32 rows 29.2 -> 24.7   48 35.0 -> 25.0   96 35.8 -> 29.4
 //               128 rows 46.6 -> 35.9  192 62.1 -> 51.8  256 74.2 -> 69.7
 //               320 rows 89.5 -> 83.4  448 117 -> 101
-constexpr int kCUs = 256;
 
 template <int TYPE, int MODE>
 static hipError_t launch_mode(const GemmArgs &a, hipStream_t s)
@@ -799,7 +925,7 @@ static hipError_t launch_mode(const GemmArgs &a, hipStream_t s)
     // One row group (the reasoning decider's rows, short branches): one wave
     // per weight row group, 1.5-2x the B-direct kernel there (12 rows of the
     // Q5_1 3B shape: 2.1 against 3.6 ms of GEMM per step)
-    if (a.M <= 16) return launch_skinny<TYPE, MODE, 4, 8>(a, s);
+    if (a.M <= 16) return launch_skinny<TYPE, MODE>(a, s);
     int tcols;           // 16-wide tile columns of the output (gate and up both count)
     bool one_seg = true; // a four-wave tile of 128 or 256 columns lies in one segment
     if (MODE == kGemmSwiGlu) {

@@ -39,16 +39,6 @@ struct RawTile {
     uint32_t qh;   // Q5_1: two bytes (block 0 low byte)
 };
 
-// Bit i of a 4-bit value x << 4 to bit 8 i + 4 (masked by the caller):
-// (x << 4) * 0x204081 (both fit 24 bits) on the full-rate 24-bit multiplier
-// (the compiler picks the quarter-rate 32-bit one for the plain product).
-__device__ __forceinline__ uint32_t spread4(uint32_t x)
-{
-    uint32_t r;
-    asm("v_mul_u32_u24 %0, %1, %2" : "=v"(r) : "v"(x), "v"(0x00204081u));
-    return r;
-}
-
 // B fragment of block bb of the tile: 8 fp16 integers for k = 8g .. 8g + 7.
 template <int TYPE>
 __device__ __forceinline__ half8_t decode_frag(const RawTile &t, int bb)
@@ -60,16 +50,9 @@ __device__ __forceinline__ half8_t decode_frag(const RawTile &t, int bb)
         bytes_to_f16(w1, (_Float16)1152.0f, o2, o3);
     } else {
         const uint32_t w = bb ? t.q.y : t.q.x;
-        uint32_t n0 = w & 0x0f0f0f0fu, n1 = (w >> 4) & 0x0f0f0f0fu;
-        _Float16 bias = (_Float16)1032.0f;
-        if (TYPE == kQ5_1) {
-            const uint32_t hb = (t.qh >> (8 * bb)) & 0xffu;
-            n0 |= spread4((hb & 15u) << 4) & 0x10101010u;
-            n1 |= spread4(hb & 0xf0u) & 0x10101010u;
-            bias = (_Float16)1024.0f;
-        }
-        bytes_to_f16(n0, bias, o0, o1);
-        bytes_to_f16(n1, bias, o2, o3);
+        if (TYPE == kQ5_1) return decode_q5_frag(w, t.qh >> (8 * bb));
+        bytes_to_f16(w & 0x0f0f0f0fu, (_Float16)1032.0f, o0, o1);
+        bytes_to_f16((w >> 4) & 0x0f0f0f0fu, (_Float16)1032.0f, o2, o3);
     }
     return __builtin_bit_cast(half8_t, make_uint4(o0, o1, o2, o3));
 }
