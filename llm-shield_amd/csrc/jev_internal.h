@@ -363,8 +363,10 @@ hipError_t launch_argmax(const float *x, int n, int32_t *result, float *scratch_
                          hipStream_t s);
 // Greedy step of the rows layout: per row, argmax(logits[r]) -> tokens[r] and
 // out[rowstep[r] * n_rows + r]; slot[r], pos[r] and rowstep[r] advance by one.
-hipError_t launch_rows_step(const float *logits, int vocab, int n_rows, int32_t *tokens, int32_t *slot, int32_t *pos,
-                            int32_t *rowstep, int32_t *out, hipStream_t s);
+// sv / si: scratch of n_rows * rows_step_parts(n_rows) entries.
+inline int rows_step_parts(int n_rows) { return n_rows >= 512 ? 1 : n_rows > 16 ? 512 / n_rows : 32; }
+hipError_t launch_rows_step(const float *logits, int vocab, int n_rows, float *sv, int32_t *si, int32_t *tokens,
+                            int32_t *slot, int32_t *pos, int32_t *rowstep, int32_t *out, hipStream_t s);
 
 // KV copy for capacity growth: [L*kvh] heads of `len` rows from stride old_cap to new_cap.
 // Pair shadow of a fp32 cache: [heads_total][cap][hd] -> [heads_total][cap][hi, lo][hd]

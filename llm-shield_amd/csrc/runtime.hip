@@ -485,8 +485,8 @@ int ensure_workspace(jev_ctx *c, int T, int n_out, int mode, int max_chunks, boo
         HIP_TRY(c->logits.ensure(nx * (size_t)f.vocab));
         if (nx >= 2) HIP_TRY(c->xt.ensure(std::max(c->xt.n, ((nx + 15) & ~(size_t)15) * f.hidden * 2)));
     }
-    HIP_TRY(c->amax_v.ensure(512));
-    HIP_TRY(c->amax_i.ensure(512));
+    HIP_TRY(c->amax_v.ensure(std::max<size_t>(512, nx))); // argmax candidates: 512, or one per output row
+    HIP_TRY(c->amax_i.ensure(std::max<size_t>(512, nx)));
     return JEV_OK;
 }
 
@@ -1879,7 +1879,8 @@ int jev_decode_rows_greedy(jev_ctx *c, int32_t shared, int32_t n_rows, const int
     auto step = [&]() -> int {
         int r = enqueue_forward(c, p, JEV_OUT_FULL, 0, c->logits.p);
         if (r) return r;
-        hipError_t e = launch_rows_step(c->logits.p, c->cfg.vocab, n_rows, const_cast<int32_t *>(p.d_tokens),
+        hipError_t e = launch_rows_step(c->logits.p, c->cfg.vocab, n_rows, c->amax_v.p, c->amax_i.p,
+                                        const_cast<int32_t *>(p.d_tokens),
                                         const_cast<int32_t *>(p.d_slot), const_cast<int32_t *>(p.d_pos), rowstep, out,
                                         c->stream);
         return e == hipSuccess ? JEV_OK : fail(JEV_EDEVICE, "rows step: %s", hipGetErrorString(e));
