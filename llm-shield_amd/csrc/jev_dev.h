@@ -48,6 +48,13 @@ __device__ __forceinline__ void split2_rtz(float x0, float x1, uint32_t &hi, uin
     lo = __builtin_bit_cast(uint32_t, l);
 }
 
+// Element i of a lane's eight quants of block bb from Q5_1's fields (QWeight).
+__device__ __forceinline__ int q5_quant(uint32_t word, uint32_t qh, int bb, int i)
+{
+    if (i < 6) return (int)((word >> (5 * (i >> 1) + 16 * (i & 1))) & 31u);
+    return (int)(((qh >> (4 * bb + 8 * (i & 1))) & 15u) | (((word >> (15 + 16 * (i & 1))) & 1u) << 4));
+}
+
 // One weight element of the tiled layout, decoded exactly as Dequantizer
 // does (Dequantizer.cs: Q4_0 :155-182, Q5_1 :240-268, Q8_0 :270-305).  d*q is
 // exact in fp32, so the Q5_1 "+ m" rounds once whether or not it is fused.
@@ -65,10 +72,12 @@ __device__ __forceinline__ float decode_elem(const QWeight &w, int row, int k)
         const int q = (int)w.qs[tile * 1024 + 16 * l + 8 * bb + i] - 128; // stored biased
         return (float)q * d;
     }
-    const uint8_t byte = w.qs[tile * 512 + 8 * l + 4 * bb + (i & 3)];
-    const int nib = i < 4 ? (byte & 15) : (byte >> 4);
-    if (type == kQ4_0) return d * (float)(nib - 8);
-    const int q = nib | (((w.qh[tile * 128 + 2 * l + bb] >> i) & 1) << 4);
+    if (type == kQ4_0) {
+        const uint8_t byte = w.qs[tile * 512 + 8 * l + 4 * bb + (i & 3)];
+        return d * (float)((i < 4 ? byte & 15 : byte >> 4) - 8);
+    }
+    const int q = q5_quant(*(const uint32_t *)(w.qs + tile * 512 + 8 * l + 4 * bb),
+                           *(const uint16_t *)(w.qh + tile * 128 + 2 * l), bb, i);
     const float m = h2f(w.d[tile * 64 + 4 * r + 2 + bb]);
     const float dq = d * (float)q;
     return dq + m;
@@ -118,28 +127,33 @@ __device__ __forceinline__ void bytes_to_f16(uint32_t bytes, _Float16 bias, uint
     p23 = sub_bias(biased_pair(bytes, 0x04030402u), bias);
 }
 
-// Bit i of a 4-bit value x << 4 to bit 8 i + 4 (masked by the caller):
-// (x << 4) * 0x204081 (both fit 24 bits) on the full-rate 24-bit multiplier
-// (the compiler picks the quarter-rate 32-bit one for the plain product).
-__device__ __forceinline__ uint32_t spread4(uint32_t x)
+// B fragment of block bb from Q5_1's fields (QWeight: word = the block's 32
+// bits, qh = the lane's 16): exact integers in [0, 31].  A quant under the
+// exponent byte at mantissa bit 0 is 1024 + q, at bit 5 1024 + 32 q, at bit 4
+// 1024 + 16 q; one packed subtraction or multiply-add leaves q.  23 vector
+// instructions per two blocks (nibbles with the fifth bits spread to the bytes
+// of a word by a multiplication took 36).
+__device__ __forceinline__ half8_t decode_q5_frag(uint32_t word, uint32_t qh, int bb)
 {
-    uint32_t r;
-    asm("v_mul_u32_u24 %0, %1, %2" : "=v"(r) : "v"(x), "v"(0x00204081u));
-    return r;
-}
-
-// A block's B fragment from Q5_1's fields: `nib` the lane's four bytes of
-// nibbles, the low byte of `qh` its fifth bits; exact integers in [0, 31].
-__device__ __forceinline__ half8_t decode_q5_frag(uint32_t nib, uint32_t qh)
-{
-    uint32_t n0 = nib & 0x0f0f0f0fu, n1 = (nib >> 4) & 0x0f0f0f0fu;
-    const uint32_t hb = qh & 0xffu;
-    n0 |= spread4((hb & 15u) << 4) & 0x10101010u;
-    n1 |= spread4(hb & 0xf0u) & 0x10101010u;
-    uint32_t o0, o1, o2, o3;
-    bytes_to_f16(n0, (_Float16)1024.0f, o0, o1);
-    bytes_to_f16(n1, (_Float16)1024.0f, o2, o3);
-    return __builtin_bit_cast(half8_t, make_uint4(o0, o1, o2, o3));
+    // in a vector register, so that mask and exponent are one v_and_or (an
+    // instruction takes one constant from the scalar side)
+    uint32_t kexp = 0x64006400u;
+    asm("" : "+v"(kexp));
+    const half2_t p0 = __builtin_bit_cast(half2_t, (word & 0x001f001fu) | kexp);
+    const half2_t p1 = __builtin_bit_cast(half2_t, (word & 0x03e003e0u) | kexp);
+    const half2_t p2 = __builtin_bit_cast(half2_t, ((word >> 10) & 0x001f001fu) | kexp);
+    const uint32_t x = biased_pair(qh, 0x04010400u); // both blocks' low bits of elements 6 | 7
+    const uint32_t y = bb ? (x & 0xfff0fff0u) | ((word >> 7) & 0x01000100u) : (x & 0xff0fff0fu) | ((word >> 11) & 0x00100010u);
+    const half2_t p3 = __builtin_bit_cast(half2_t, y);
+    auto scaled = [](half2_t v, _Float16 r) { // (1024 + n q) / n - 1024 / n, r = 1 / n
+        const _Float16 c = (_Float16)-1024.0f * r;
+        return __builtin_elementwise_fma(v, half2_t{r, r}, half2_t{c, c});
+    };
+    const half2_t k = {(_Float16)1024.0f, (_Float16)1024.0f};
+    const half2_t o0 = p0 - k, o1 = scaled(p1, (_Float16)0.03125f), o2 = p2 - k,
+                  o3 = bb ? scaled(p3, (_Float16)0.0625f) : p3 - k;
+    return __builtin_bit_cast(half8_t, make_uint4(__builtin_bit_cast(uint32_t, o0), __builtin_bit_cast(uint32_t, o1),
+                                                  __builtin_bit_cast(uint32_t, o2), __builtin_bit_cast(uint32_t, o3)));
 }
 
 __device__ __forceinline__ float warp_sum(float v)

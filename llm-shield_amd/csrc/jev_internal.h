@@ -27,13 +27,18 @@ int64_t row_bytes(int type, int64_t cols);
 // an even count with zero quants and scales.  Per tile:
 //   qs  Q8_0       1024 B: lane l's 16 bytes at 16 l -- 8 quants of block 0, then 8 of block 1,
 //                          each stored biased as the byte q + 128
-//       Q4_0/Q5_1   512 B: lane l's 8 bytes at 8 l -- 4 of block 0, then 4 of block 1; byte i
+//       Q4_0        512 B: lane l's 8 bytes at 8 l -- 4 of block 0, then 4 of block 1; byte i
 //                          of a block's four = element 8g+i (low nibble) | element 8g+i+4 (high)
+//       Q5_1        512 B: lane l's 8 bytes at 8 l, a 32-bit word per block: element 8g+i, i < 6,
+//                          at bits 5 (i / 2) + 16 (i % 2) .. + 4, the fifth bits of elements
+//                          8g+6 and 8g+7 at bits 15 and 31 -- even elements in the low half, odd
+//                          ones in the high half, so a mask and an exponent make an fp16 pair
 //   d   fp16         64 B: row r's two block scales at 4 r (Q8_0, Q4_0)
 //       Q5_1        128 B: row r's two scales then its two mins at 8 r, so a
 //                          lane's scales and mins are one 8-byte load
 //                          (QWeight::m points at the first min)
-//   qh  (Q5_1)      128 B: lane l's fifth bits at 2 l + block, bit i = element 8 g + i
+//   qh  (Q5_1)      128 B: lane l's 16 bits at 2 l -- the low four bits of elements 8g+6 (at 4 block)
+//                          and 8g+7 (at 8 + 4 block)
 //   qb  (Q5_1)     1024 B: the same quants again as whole bytes q in [0, 31], in
 //                          Q8_0's order (lane l's 16 bytes at 16 l), for the
 //                          kernels of two or more tokens: one byte permute and

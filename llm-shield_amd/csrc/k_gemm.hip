@@ -692,7 +692,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_skinny_kernel(GemmArgs a, int
         for (int n = 0; n < TN; n++) {
             half8_t bf;
             if constexpr (F5)
-                bf = decode_q5_frag(bb ? s.b[n].q.y : s.b[n].q.x, s.qh[n] >> (8 * bb));
+                bf = decode_q5_frag(bb ? s.b[n].q.y : s.b[n].q.x, s.qh[n], bb);
             else
                 bf = decode_b_frag<TYPE>(s.b[n], bb);
             Pair t;

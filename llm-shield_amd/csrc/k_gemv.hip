@@ -8,7 +8,7 @@
 //
 //  * x (fp32) is split once per workgroup into an fp16 pair x = hi + lo
 //    (~22 significant bits) and staged in LDS.  It is the MFMA A operand:
-//    row 0 holds hi, row 1 holds lo, rows 2..15 read a zero slot.
+//    row 0 holds hi, row 1 holds lo, rows 2..15 read zeros.
 //  * A wave owns 16 weight rows, one tile row of the tiled weight layout.
 //    Per tile (two quant blocks) a lane loads its slot -- the quants of its
 //    row (l % 16) at k = 8 (l / 16) .. + 7 of both blocks, exactly its B
@@ -17,6 +17,12 @@
 //  * One v_mfma_f32_16x16x32_f16 per block then yields x_hi . q and x_lo . q
 //    for the 16 rows; the fp32 scale is applied on the vector ALU:
 //    acc += d * (p_hi + p_lo)  (+ m * sum(x) over the block for Q5_1).
+//
+// Q5_1, cold weights, us, before -> with 23 instead of 36 decode instructions
+// per tile, x addressed by a masked add per stage, and the scale FMAs one block
+// behind their MFMA: QKV 5.3 -> 5.0, O 4.9 -> 4.7, down 8.0 -> 7.2, gate/up
+// 12.9 -> 12.4, head 62.5 -> 60.0 (5.0 TB/s; Q8_0's head, two load streams
+// instead of three, 5.8).
 //
 // Narrow projections split K over the workgroup's four waves and, for more
 // parallelism, over `ksplit` workgroups whose partials land ksplit * N floats
@@ -31,12 +37,12 @@ namespace jev {
 namespace {
 
 
-// One lane's share of a tile: its quants for both blocks, the two scales /
-// mins of its row and its fifth bits.
+// One lane's share of a tile: its quants for both blocks and the two scales /
+// mins of its row.
 struct RawTile {
     uint4 q;       // Q8_0: 16 bytes; Q4_0 / Q5_1: 8 bytes in .x, .y
     uint32_t d, m; // two fp16 each (block 0 low half)
-    uint32_t qh;   // Q5_1: two bytes (block 0 low byte)
+    uint32_t qh;   // Q5_1: QWeight::qh's 16 bits of the lane
 };
 
 // B fragment of block bb of the tile: 8 fp16 integers for k = 8g .. 8g + 7.
@@ -50,7 +56,7 @@ __device__ __forceinline__ half8_t decode_frag(const RawTile &t, int bb)
         bytes_to_f16(w1, (_Float16)1152.0f, o2, o3);
     } else {
         const uint32_t w = bb ? t.q.y : t.q.x;
-        if (TYPE == kQ5_1) return decode_q5_frag(w, t.qh >> (8 * bb));
+        if (TYPE == kQ5_1) return decode_q5_frag(w, t.qh, bb);
         bytes_to_f16(w & 0x0f0f0f0fu, (_Float16)1032.0f, o0, o1);
         bytes_to_f16((w >> 4) & 0x0f0f0f0fu, (_Float16)1032.0f, o2, o3);
     }
@@ -185,10 +191,13 @@ __global__ __launch_bounds__(256, 2) void gemv_q_kernel(GemvArgs a, int nrows, i
     }
     load_stage(0, r0);
 
-    // ---- x pair of the workgroup's K range (zero past K), a zero slot, Q5_1 block sums
+    // ---- x pair of the workgroup's K range (zero past K), zeros, Q5_1 block
+    // sums.  A wave's last stage may read up to DEPTH - 1 tiles past its range
+    // (against zero weights): a neighbour's, or zeros.
     uint16_t *xh = (uint16_t *)smem, *xl = xh + nbz * 32, *zero = xl + nbz * 32;
-    float *xsum = (float *)(zero + 8);
-    float *red = xsum + nbz; // [4][NW][16] wave partials
+    constexpr int kZero = DEPTH * 64 > 256 ? DEPTH * 64 : 256; // halves: a stage of zeros, the wave partials later
+    float *xsum = (float *)(zero + kZero);
+    float *red = (float *)zero; // [4][NW][16] wave partials, once the zeros are read
     // decode attention input: the token's chunk count, as the attention
     // kernel computes it
     int nch = 0;
@@ -299,39 +308,64 @@ __global__ __launch_bounds__(256, 2) void gemv_q_kernel(GemvArgs a, int nrows, i
     stage_group(0, std::integral_constant<int, ATTN ? -1 : 0>{});
     if (256 < 2 * ntw * 4) stage_group(256, std::integral_constant<int, ATTN ? -1 : 1>{});
     for (int i0 = 256 * kPre; i0 < 2 * ntw * 4; i0 += 256) stage_group(i0, std::integral_constant<int, -1>{});
-    if (tid < 8) zero[tid] = 0;
+    for (int i = tid; i < kZero / 8; i += 256) *(uint4 *)(zero + 8 * i) = make_uint4(0u, 0u, 0u, 0u);
+    if (tid < 8 * (DEPTH - 1)) {
+        const int i = 2 * ntw * 4 + tid; // the tiles past the range
+        if (i < nbz * 4) {
+            *(uint4 *)(xh + 8 * i) = make_uint4(0u, 0u, 0u, 0u);
+            *(uint4 *)(xl + 8 * i) = make_uint4(0u, 0u, 0u, 0u);
+        }
+        if (TYPE == kQ5_1 && (tid & 3) == 0) xsum[i >> 2] = 0.f;
+    }
     __syncthreads();
 
-    // A fragment address: row 0 -> hi, row 1 -> lo, rows 2..15 -> the zero slot
-    const uint16_t *abase = rl == 0 ? xh + 8 * g : rl == 1 ? xl + 8 * g : zero;
-    const int astep = rl <= 1 ? 32 : 0;
+    // A fragment address: row 0 -> hi, row 1 -> lo, rows 2..15 -> the zeros.
+    // One masked add per stage; its tiles and blocks are offsets in the reads
+    // (a multiplication and two additions per tile before).
+    const uint32_t aoff = rl == 0 ? 16 * g : rl == 1 ? nbz * 64 + 16 * g : nbz * 128;
+    const uint32_t amask = rl <= 1 ? ~0u : 0u;
 
     float acc[NW];
 #pragma unroll
     for (int w = 0; w < NW; w++) acc[w] = 0.f;
 
+    struct Late { // a block's products and what scales them
+        floatx4 p;
+        float d, m, xs;
+    };
+    auto apply = [&](int w, const Late &t) __attribute__((always_inline)) {
+        acc[w] = fmaf(t.d, t.p[0] + t.p[1], acc[w]);
+        if (TYPE == kQ5_1) acc[w] = fmaf(t.m, t.xs, acc[w]);
+    };
     auto compute_stage = [&](int st, const RawTile (&r)[NW][DEPTH]) {
+        const int lt = t0 + st * DEPTH; // the stage's first tile within the workgroup's range
+        const uint8_t *ap = smem + (aoff + ((uint32_t)(lt * 128) & amask));
+        const float *xs = xsum + 2 * lt;
+        // each block's scale FMAs after the next block's MFMA: they need not
+        // wait for the matrix core
+        Late late[NW];
 #pragma unroll
         for (int j = 0; j < DEPTH; j++) {
-            const int tl = st * DEPTH + j; // tile within the wave's range
-            const int lt = t0 + min(tl, ntiles - 1); // tile within the workgroup's range
 #pragma unroll
             for (int bb = 0; bb < 2; bb++) {
-                const half8_t af = *(const half8_t *)(abase + astep * (2 * lt + bb));
+                const half8_t af = *(const half8_t *)(ap + 128 * j + 64 * bb);
 #pragma unroll
                 for (int w = 0; w < NW; w++) {
                     const half8_t bf = decode_frag<TYPE>(r[w][j], bb);
-                    floatx4 p = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    const float dv = half_of(r[w][j].d, bb); // 0 past the range
-                    const float v = p[0] + p[1];
-                    acc[w] = fmaf(dv, v, acc[w]);
+                    Late t;
+                    t.p = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    t.d = half_of(r[w][j].d, bb); // 0 past the range
                     if (TYPE == kQ5_1) {
-                        const float mv = half_of(r[w][j].m, bb);
-                        acc[w] = fmaf(mv, xsum[2 * lt + bb], acc[w]);
+                        t.m = half_of(r[w][j].m, bb);
+                        t.xs = xs[2 * j + bb];
                     }
+                    if (j > 0 || bb > 0) apply(w, late[w]);
+                    late[w] = t;
                 }
             }
         }
+#pragma unroll
+        for (int w = 0; w < NW; w++) apply(w, late[w]);
     };
 
     // Two register stages; whole pairs in the loop, the odd stage after it.
@@ -358,6 +392,7 @@ __global__ __launch_bounds__(256, 2) void gemv_q_kernel(GemvArgs a, int nrows, i
     if (WR == 4) {
         if (g == 0 && row < nrows) a.y[(size_t)z * nrows + row] = acc[0];
     } else {
+        __syncthreads(); // the zeros are read
         if (g == 0) {
 #pragma unroll
             for (int w = 0; w < NW; w++) red[(wave * NW + w) * 16 + rl] = acc[w];
@@ -388,7 +423,9 @@ static hipError_t launch_gemv_cfg(const GemvArgs &a, int rows, hipStream_t s)
     const int nb = a.K >> 5;
     const int nbz = gemm_split_blocks(nb, a.ksplit);
     const int groups = (rows + 15) / 16;
-    size_t lds = (size_t)nbz * 32 * 2 * 2 + 16 + (size_t)nbz * 4 + 4 * 2 * 16 * 4; // nbz is even
+    // x pair, zeros (of a four-tile stage, the larger), block sums of the range
+    // and of three tiles past it; nbz is even
+    size_t lds = (size_t)nbz * 32 * 2 * 2 + 4 * 64 * 2 + (size_t)nbz * 4 + 6 * 4;
     if (lds > 64 * 1024) return hipErrorInvalidValue;
     dim3 grid(WR == 4 ? (groups + 3) / 4 : groups, a.ksplit);
     // tiles of one wave, and the stage depth that pads them least (4 on a tie)

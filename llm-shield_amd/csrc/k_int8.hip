@@ -210,7 +210,7 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_kernel(GemmI8Args a)
     // ---- weight slot of tile pair kp (clamped past the last)
     struct WStage {
         uint4 q;     // Q8_0 16 bytes, nibbles 8 in .x, .y
-        uint32_t qh; // Q5_1 fifth bits (block 0 low byte)
+        uint32_t qh; // Q5_1: QWeight::qh's 16 bits of the lane
         uint2 dm;    // two scales (.x; Q5_1: mins in .y)
     };
     auto load_w = [&](WStage &s, int kp) __attribute__((always_inline)) {
@@ -251,14 +251,17 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_kernel(GemmI8Args a)
 #pragma unroll
             for (int bb = 0; bb < 2; bb++) {
                 const uint32_t v = bb ? s.q.y : s.q.x;
-                uint32_t n0 = v & 0x0f0f0f0fu, n1 = (v >> 4) & 0x0f0f0f0fu;
                 if (TYPE == kQ5_1) {
-                    const uint32_t hb = (s.qh >> (8 * bb)) & 0xffu;
-                    n0 |= (((hb & 15u) * 0x00204081u) & 0x01010101u) << 4;
-                    n1 |= (((hb >> 4) * 0x00204081u) & 0x01010101u) << 4;
+                    // element pairs (QWeight's word: 0 | 1, 2 | 3, 4 | 5; 6 | 7 with qh)
+                    const uint32_t p0 = v & 0x001f001fu, p1 = (v >> 5) & 0x001f001fu, p2 = (v >> 10) & 0x001f001fu;
+                    const uint32_t lo = __builtin_amdgcn_perm(0u, s.qh, 0x0c010c00u) >> (4 * bb); // bytes 0 and 2
+                    const uint32_t p3 = (lo & 0x000f000fu) | ((v >> 11) & 0x00100010u);
+                    wq[bb][0] = __builtin_amdgcn_perm(p1, p0, 0x06040200u);
+                    wq[bb][1] = __builtin_amdgcn_perm(p3, p2, 0x06040200u);
+                } else {
+                    wq[bb][0] = v & 0x0f0f0f0fu;
+                    wq[bb][1] = (v >> 4) & 0x0f0f0f0fu;
                 }
-                wq[bb][0] = n0;
-                wq[bb][1] = n1;
             }
         }
 #pragma unroll

@@ -52,11 +52,10 @@ __global__ __launch_bounds__(256) void gather_kernel(QWeight w, const int32_t *i
                 }
             } else {
                 const float d = h2f(w.d[tile * 64 + 4 * r + bb]), m = h2f(w.d[tile * 64 + 4 * r + 2 + bb]);
-                const uint32_t qh = w.qh[tile * 128 + 2 * l + bb];
+                const uint32_t qh = *(const uint16_t *)(w.qh + tile * 128 + 2 * l);
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
-                    const int nib = (int)((q >> (8 * (i & 3) + (i < 4 ? 0 : 4))) & 15u);
-                    const int qi = nib | (int)(((qh >> i) & 1u) << 4);
+                    const int qi = q5_quant(q, qh, bb, i);
                     const float dq = d * (float)qi;
                     v[i] = dq + m;
                 }

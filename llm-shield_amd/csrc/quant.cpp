@@ -165,22 +165,25 @@ bool repack_host(int type, int64_t rows, int64_t cols, const void *gguf, void *d
                     std::memcpy(out + L.d + tile * dstride + drow * r + 4 + 2 * bb, blk + 2, 2);
                     std::memcpy(&qh, blk + 4, 4);
                 }
+                auto nib = [&](int j) { return (uint32_t)(j < 16 ? (qs[j] & 15) : (qs[j - 16] >> 4)); };
                 for (int g = 0; g < 4; g++) {
-                    uint8_t *dq = out + L.qs + tile * TQ + 8 * (16 * g + r) + 4 * bb;
-                    for (int i = 0; i < 4; i++) {
-                        auto nib = [&](int j) { return j < 16 ? (qs[j] & 15) : (qs[j - 16] >> 4); };
-                        dq[i] = (uint8_t)(nib(8 * g + i) | (nib(8 * g + i + 4) << 4));
+                    const size_t lane = 16 * g + r;
+                    uint8_t *dq = out + L.qs + tile * TQ + 8 * lane + 4 * bb;
+                    if (type == kQ4_0) {
+                        for (int i = 0; i < 4; i++) dq[i] = (uint8_t)(nib(8 * g + i) | (nib(8 * g + i + 4) << 4));
+                        continue;
                     }
-                    if (type == kQ5_1) {
-                        out[L.qh + tile * 128 + 2 * (16 * g + r) + bb] = (uint8_t)((qh >> (8 * g)) & 0xffu);
-                        // the byte copy: element 8 g + i at byte 8 bb + i of lane 16 g + r
-                        uint8_t *db = out + L.qb + tile * 1024 + 16 * (16 * g + r) + 8 * bb;
-                        for (int i = 0; i < 8; i++) {
-                            const int j = 8 * g + i;
-                            const int nibj = j < 16 ? (qs[j] & 15) : (qs[j - 16] >> 4);
-                            db[i] = (uint8_t)(nibj | (((qh >> j) & 1u) << 4));
-                        }
-                    }
+                    uint32_t q[8], word = 0;
+                    for (int i = 0; i < 8; i++) q[i] = nib(8 * g + i) | (((qh >> (8 * g + i)) & 1u) << 4);
+                    for (int i = 0; i < 6; i++) word |= q[i] << (5 * (i / 2) + 16 * (i % 2));
+                    word |= (q[6] >> 4) << 15 | (q[7] >> 4) << 31;
+                    std::memcpy(dq, &word, 4);
+                    uint8_t *lo = out + L.qh + tile * 128 + 2 * lane;
+                    lo[0] |= (uint8_t)((q[6] & 15u) << (4 * bb));
+                    lo[1] |= (uint8_t)((q[7] & 15u) << (4 * bb));
+                    // the byte copy: element 8 g + i at byte 8 bb + i of lane 16 g + r
+                    uint8_t *db = out + L.qb + tile * 1024 + 16 * lane + 8 * bb;
+                    for (int i = 0; i < 8; i++) db[i] = (uint8_t)q[i];
                 }
             }
         }
