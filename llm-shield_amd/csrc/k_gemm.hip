@@ -978,15 +978,41 @@ static hipError_t launch_mode(const GemmArgs &a, hipStream_t s)
         if constexpr (TYPE == kQ5_1) return launch_bd<TYPE, MODE, 4, 1, 1, 1, false, 8>(a, s);
         return launch_bd<TYPE, MODE, 2, 2, 1, 1, false, 8>(a, s);
     }
-    // Large batches.  Four-wave 64 x 256 tiles keep 16 tiles per wave, and
-    // with them Q5_1 has no registers for its byte quants: eight waves of 64 x
-    // 32 there at every size.
+    // Large batches, tiles of 256 columns.
     if constexpr (MODE == kGemmStore && TYPE != kQ5_1)
         if (a.fold) return launch_bd<TYPE, MODE, 4, 4, 1, 2, true>(a, s);
-    if (TYPE == kQ5_1 || !one_seg || (MODE == kGemmStore && wgs(4, 2, 8) <= 2 * kCUs))
-        return launch_bd<TYPE, MODE, 4, 2, 1, 1, false, 8>(a, s);
-    if constexpr (TYPE != kQ5_1) return launch_bd<TYPE, MODE, 4, 4, 1, 2>(a, s);
-    return hipErrorInvalidValue; // not reached
+    // The height of the tile by the rounds its grid takes.  Eight waves of 64,
+    // 80 or 96 rows x 32 columns (two such workgroups fit a CU) finish when the
+    // busiest CU does, so their time is whole workgroups per CU times a
+    // workgroup's; four waves of 64 x 64, two workgroups at a time, run on
+    // through a partial round, and past four rounds, where the power limit sets
+    // the clock, are the cheapest per row.  Relative times per workgroup from
+    // launches of 520 to 3000 rows (us, 64 rows / 80 / 96 / the four waves): Q8_0
+    // O, 700 rows 49.3 / 42.4 / 46.6 / 48.5, 900 52.4 / 62.3 / 50.4 / 52.1, 1500 82.2 /
+    // 83.5 / 77.6 / 82.1; SwiGLU, 520 rows 141 / 125 / 135 / 141, 900 238 / 237 / 213 /
+    // 251.  Q5_1 has no registers for 96 rows, nor for its byte quants in the
+    // four-wave tile.
+    constexpr double k80 = TYPE == kQ8_0 ? 1.26 : TYPE == kQ4_0 ? 1.34 : MODE == kGemmStore ? 1.31 : 1.48, k96 = 1.42;
+    auto rounds = [&](int tm) { return (double)((wgs(tm, 2, 8) + kCUs - 1) / kCUs); };
+    double best = rounds(4);
+    int tall = 4;
+    if (rounds(5) * k80 < best) {
+        best = rounds(5) * k80;
+        tall = 5;
+    }
+    if constexpr (TYPE != kQ5_1) {
+        if (rounds(6) * k96 < best) {
+            best = rounds(6) * k96;
+            tall = 6;
+        }
+        const double share = (double)wgs(4, 4, 4) / kCUs, r4 = rounds(4);
+        const double four = (share == r4 ? r4 : share + 0.85) * (share > 4 ? 0.95 : 0.98);
+        if (one_seg && (four < best || (tall == 4 && share > 4)) && (MODE == kGemmSwiGlu || r4 > 2))
+            return launch_bd<TYPE, MODE, 4, 4, 1, 2>(a, s);
+        if (tall == 6) return launch_bd<TYPE, MODE, 6, 2, 1, 4, false, 8>(a, s);
+    }
+    if (tall == 5) return launch_bd<TYPE, MODE, 5, 2, 1, 4, false, 8>(a, s);
+    return launch_bd<TYPE, MODE, 4, 2, 1, 1, false, 8>(a, s);
 }
 
 template <int TYPE>

@@ -42,3 +42,29 @@ def test_prompt_rows_do_not_depend_on_the_prompt_length(gpu, t):
             seen = got
         assert np.array_equal(seen, got), n
     model.close()
+
+
+@pytest.mark.parametrize("t", TYPES)
+def test_matmul_rows_do_not_depend_on_the_height_of_a_large_batch_tile(gpu, t):
+    rows, cols = 3060, 2112
+    raw = jev.synth_tensor("tall", t, rows, cols)
+    x = np.random.default_rng(6).standard_normal((1700, cols)).astype(np.float32)
+    full = matmul_gpu(t, raw, rows, cols, x, 1700)
+    # 80-row tiles at 700, 96-row at 900 and 1500, 64-row between
+    for n in (641, 700, 720, 721, 768, 900, 960, 961, 1100, 1500, 1536, 1537):
+        lo = (n * 7) % (1700 - n)
+        assert np.array_equal(full[lo:lo + n], matmul_gpu(t, raw, rows, cols, x[lo:lo + n], n)), n
+
+
+@pytest.mark.parametrize("t", TYPES)
+def test_prompt_rows_do_not_depend_on_a_longer_prompt_s_tiles(gpu, t):
+    cfg = jev.ModelConfig(n_layers=1, vocab=512, initial_kv_capacity=1100)
+    model = jev.SynthModel(cfg, t).open(0)
+    tokens = jev.random_tokens(1024, cfg.vocab, 8)
+    seen = None
+    for n in (17, 520, 560, 561, 576, 700, 720, 900, 960, 961, 1024):
+        model.reset_kv_cache()
+        got = model.forward_layout(tokens[:n], jev.TokenLayout.tree(0, n, [], n).with_outputs([2, 9, 16]), jev.OUT_FULL)
+        seen = got if seen is None else seen
+        assert np.array_equal(seen, got), n
+    model.close()
