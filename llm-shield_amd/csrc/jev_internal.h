@@ -268,11 +268,15 @@ struct AttnTile {
     int32_t t0, n, shared_lo, shared_hi, segment, slot0, pad0, pad1;
 };
 // Logical key blocks (of 64) per partition: a tile's online softmax restarts
-// at every partition and the partitions merge in ascending order.  512 keys
-// are the largest power of two that still spreads a 4096-token context over
-// the GPU for a handful of queries; the merge costs a tile ~3 % of a
-// partition's own time.
-constexpr int kAttnPartBlocks = 8;
+// at every partition and the partitions merge in ascending order.  A merge
+// costs a tile ~1200 cycles beside a block's 5400, so with 512 keys prompts of
+// 600 to 4500 tokens lost 2-5 % of their attention (1000 tokens 44.5 -> 47.5 us
+// a layer in the model); with 1024 keys up to that many pay nothing and longer
+// ones half, and passes of a few hundred queries, whose partials weigh more,
+// gain (600 tokens over 4096 cached 160 -> 141 us).  A handful of queries over a
+// long context would take the smaller ones (30 tokens over 4096: 25 us against
+// 34; whole, 102).
+constexpr int kAttnPartBlocks = 16;
 constexpr int kAttnPartFloats = 64 + 32 * 128; // one tile and head's partial: 32 maxima, 32 sums, 32 x 128 outputs
 // How a pass's attention is cut into workgroups: ds of them per (tile, KV
 // head) share the output dims, and with run_blocks > 0 every run of that many

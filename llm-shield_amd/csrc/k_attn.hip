@@ -31,8 +31,8 @@
 //   O^T (128 x 32) += V^T (128 x 64) . P^T (64 x 32)      48 MFMAs per 64 keys,
 //                     keys taken in the order the S^T fragments hold them
 //
-// Partitions.  The blocks form partitions of kAttnPartBlocks (512 logical
-// keys), each its own online softmax from scratch, and the partitions' (max,
+// Partitions.  The blocks form partitions of kAttnPartBlocks (1024
+// logical keys), each its own online softmax from scratch, and the partitions' (max,
 // sum, o) are merged in ascending order: a rule on the logical key index alone,
 // so a query's arithmetic still does not depend on what runs beside it, and a
 // partition may run in any workgroup.  A pass whose tiles and heads fill the
@@ -130,13 +130,19 @@ __device__ __forceinline__ half8_t cat4(uint2 a, uint2 b)
 // The operations and their order per output are those of the plain sequence
 // S(b), P V(b - 1), softmax(b), rescale, so the bits do not depend on it.
 //
-// SPLIT: blockIdx.z also counts runs of a.run_blocks blocks (whole
-// partitions); the workgroup walks its run and stores each partition's (max,
-// sum, o) instead of merging them.
-template <int DS, bool SPLIT>
+// PARTS: how the partitions of kAttnPartBlocks blocks come together.  kOnePart:
+// no tile has a second one, and neither its registers nor its code is there
+// (24 us against 25.4 for 750 tokens of five-option decisions: the launch is
+// short enough for the fetch of its instructions to show).  kMerged: the
+// workgroup merges them as it goes.  kSplit: blockIdx.z also counts runs of
+// a.run_blocks blocks (whole partitions); the workgroup walks its run and
+// stores each partition's (max, sum, o) for attn_merge_kernel.
+enum AttnParts { kOnePart, kMerged, kSplit };
+template <int DS, int PARTS>
 __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
 {
     constexpr int ND = 4 / DS; // 32-dim output tiles per wave
+    constexpr bool SPLIT = PARTS == kSplit, MERGE = PARTS == kMerged;
     // Double-buffered K and V blocks as fp16 pairs: [key][hi, lo][16 chunks of
     // 8 dims], chunks swizzled per key (chunk ^ swz(key)) so that both the
     // K fragment reads and the V transpose reads hit distinct banks.  One
@@ -373,7 +379,7 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
         if (k == MNEW) {
             // a partition's first block starts from scratch: alpha is 0
             m_old = m_run;
-            const float mp = b % kAttnPartBlocks == 0 ? -INFINITY : m_run;
+            const float mp = PARTS != kOnePart && b % kAttnPartBlocks == 0 ? -INFINITY : m_run;
             m_new = fmaxf(mp, fmaxf(bmax, bmax_o));
             m_run = m_new;
             // a query that sees nothing of its partition yet: exponentials of -inf - 0
@@ -427,7 +433,6 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
 
     // The finished partitions' merge, in accumulation registers (one workgroup
     // for the whole tile) or in memory (SPLIT).
-    constexpr bool MERGE = !SPLIT;
     floatx16 ot[MERGE ? ND : 1];
     float m_tot = -INFINITY, l_tot = 0.f;
     if constexpr (MERGE) {
@@ -453,7 +458,7 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
                 for (int j = 0; j < 16; j++) ot[d][j] = fmaf(o[d][j], fp, ot[d][j] * fo);
                 asm volatile("" : "+a"(ot[d]));
             }
-        } else if (q_ok) {
+        } else if (SPLIT && q_ok) {
             // [tile][head][partition]: the 32 queries' maxima, their sums, then
             // o as [dim / 4][query][4] (32 lanes store 512 contiguous bytes)
             float *pp = a.part + (((size_t)(a.n_tiles - 1 - (int)blockIdx.y) * a.n_heads + head) * a.n_parts + p) * kAttnPartFloats;
@@ -502,7 +507,7 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
     };
     // block b is the first of a partition: the one before it is complete in o
     // once P V(b - 1) has run, which is before step b + 1
-    auto opens = [&](int b) { return b > b0 && b % kAttnPartBlocks == 0; };
+    auto opens = [&](int b) { return PARTS != kOnePart && b > b0 && b % kAttnPartBlocks == 0; };
     for (int b = b0 + 1; b < b1; b += 2) {
         if (opens(b - 1)) end_part((b - 1) / kAttnPartBlocks - 1, m_old);
         if (tail(b))
@@ -528,13 +533,16 @@ __global__ __launch_bounds__(256, 1) void attn_tree_kernel(AttnArgs a)
         end_part((b1 - 1) / kAttnPartBlocks, m_run);
         return;
     }
-    if (b1 > kAttnPartBlocks) { // several partitions: their merge
-        end_part(0, m_run);
-        if constexpr (MERGE) {
+    if constexpr (MERGE) {
+        if (b1 > kAttnPartBlocks) { // several partitions: the last one's merge
+            const float mn = fmaxf(m_tot, m_run);
+            const float fo = __builtin_amdgcn_exp2f(m_tot - mn), fp = __builtin_amdgcn_exp2f(m_run - mn);
+            l_run = fmaf(l_run, fp, l_tot * fo);
 #pragma unroll
-            for (int d = 0; d < ND; d++) o[d] = ot[d];
+            for (int d = 0; d < ND; d++)
+#pragma unroll
+                for (int j = 0; j < 16; j++) o[d][j] = fmaf(o[d][j], fp, ot[d][j] * fo);
         }
-        l_run = l_tot;
     }
     if (q_ok) {
         // o[d][j] is dim 32 (ND dh + d) + 8 (j / 4) + 4 g + j % 4: four
@@ -608,10 +616,10 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a)
 // workgroup (128 KiB of LDS) runs per compute unit; a split pass pays the merge
 // launch and writes and reads its partials (~4 TB/s).  Measured (32 / 8 heads,
 // us per layer, one workgroup per tile and head group with the grid's ds
-// against this choice): 30 tokens over 4096 cached 106 -> 27, over 1100 33 ->
-// 21; 300 over 4096 124 -> 79, over 2000 67 -> 47; 5 options of 13 over 2000 57
-// -> 29; 9 options of 48 over 4096 250 (two rounds of ds 2) -> 141 (one of ds
-// 1); a 4096-token prompt's own tiles stay whole.
+// against this choice): 30 tokens over 4096 cached 102 -> 34, over 2000 53 -> 33;
+// 300 over 4096 121 -> 80, over 2000 66 -> 45; 600 over 4096 155 -> 141, over 1100
+// 61 -> 51; 5 options of 13 over 2000 58 -> 38; 9 options of 48 over 4096 250 (two
+// rounds of ds 2) -> 138; a 4096-token prompt's own tiles stay whole.
 AttnSchedule attn_schedule(int n_tiles, int n_heads, int group, int max_blocks, double total_blocks)
 {
     constexpr int kCUs = 256;
@@ -667,15 +675,19 @@ hipError_t launch_attn_tree(const AttnArgs &args, hipStream_t s)
     const int runs = c.run_blocks > 0 ? (c.n_parts * kAttnPartBlocks + c.run_blocks - 1) / c.run_blocks : 1;
     const dim3 grid(n_kv * hsets, a.n_tiles, c.ds * runs);
     auto launch = [&](auto kernel) { launch_stamped(a.ev_start, a.ev_stop, kernel, grid, dim3(256), 0, s, a); };
+    auto launch_ds = [&](auto parts) {
+        constexpr int P = decltype(parts)::value;
+        if (c.ds == 4) launch(attn_tree_kernel<4, P>);
+        else if (c.ds == 2) launch(attn_tree_kernel<2, P>);
+        else launch(attn_tree_kernel<1, P>);
+    };
     if (c.run_blocks > 0) {
-        if (c.ds == 4) launch(attn_tree_kernel<4, true>);
-        else if (c.ds == 2) launch(attn_tree_kernel<2, true>);
-        else launch(attn_tree_kernel<1, true>);
+        launch_ds(std::integral_constant<int, kSplit>{});
         hipLaunchKernelGGL(attn_merge_kernel, dim3(a.n_heads, a.n_tiles), dim3(256), 0, s, a);
+    } else if (c.n_parts > 1) {
+        launch_ds(std::integral_constant<int, kMerged>{});
     } else {
-        if (c.ds == 4) launch(attn_tree_kernel<4, false>);
-        else if (c.ds == 2) launch(attn_tree_kernel<2, false>);
-        else launch(attn_tree_kernel<1, false>);
+        launch_ds(std::integral_constant<int, kOnePart>{});
     }
     return hipGetLastError();
 }

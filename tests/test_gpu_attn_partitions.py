@@ -1,4 +1,4 @@
-"""Attention over several 512-key partitions: split across workgroups (few queries
+"""Attention over several 1024-key partitions: split across workgroups (few queries
 over a long context) and merged inside one (many), the bits do not depend on which,
 and both match the oracle."""
 import numpy as np
