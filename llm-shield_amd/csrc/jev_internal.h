@@ -351,6 +351,13 @@ struct AttnCombineArgs {
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
 };
 hipError_t launch_attn_combine(const AttnCombineArgs &a, hipStream_t s);
+// One token's decode attention combined into out [n_heads * 128] (the O GEMV's
+// plain input) when its context may have more than kCombineChunks chunks: the
+// GEMV's workgroups each merge the chunks of their K range, 768 of them reading
+// what one workgroup per head here reads once (Q8_0 O in the model, us, inside ->
+// ahead: 93 chunks 24.4 -> 11.6, 63 18.3 -> 9.9, 24 10.3 -> 8.9; 9, Q5_1, 8.1 -> 8.2).
+constexpr int kCombineChunks = 16;
+hipError_t launch_attn_combine_one(const DecodeChunks &d, int n_heads, float *out, hipStream_t s);
 
 // Verdict-row head: for each output b, logits[b][i] = dot(norm(h[outputs[b]]), W[rows[i]]).
 struct HeadRowsArgs {

@@ -1082,4 +1082,77 @@ hipError_t launch_attn_combine(const AttnCombineArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
+// One token's chunks combined ahead of the O projection's GEMV: one workgroup per
+// head, with the operations the GEMV applies while staging its input, so the
+// same bits.  64 chunks at a time come into LDS in one round of loads; lane c of
+// the first wave forms chunk c's two factors (the running max before it and with
+// it are prefix maxima, exact in any order), and thread d of 128 runs dim d's
+// chain over them.  (One wave per head that loaded chunk by chunk took 11.9 us
+// for 63 chunks, its loads' latencies.)
+__global__ __launch_bounds__(256) void attn_combine_one_kernel(DecodeChunks d, float *out)
+{
+    constexpr int NC = 64, ROW = 65; // chunks at a time, a chunk's (max, sum, o[128]) in float2
+    __shared__ __attribute__((aligned(16))) float2 part[NC * ROW];
+    __shared__ float fo[NC], fc[NC];
+    const int h = blockIdx.x, tid = threadIdx.x;
+    const int start = d.start_dev ? *d.start_dev : d.start;
+    const int slot = d.slot ? d.slot[0] : start;
+    const int slo = d.shared_lo ? d.shared_lo[0] : 0;
+    const int shi = d.shared_hi ? d.shared_hi[0] : start;
+    const int seg = d.segment ? d.segment[0] : start;
+    const int limit = (shi - slo) + (slot - seg + 1);
+    const int nch = min((limit + kDecodeKeys - 1) / kDecodeKeys, d.max_chunks);
+    const float2 *pp = (const float2 *)(d.part + (size_t)h * d.max_chunks * 2 * ROW);
+    float M = -INFINITY, L = 0.f, v = 0.f;
+    for (int c0 = 0; c0 < nch; c0 += NC) {
+        const int n = min(NC, nch - c0);
+        constexpr int B = (NC * ROW + 255) / 256;
+        float2 buf[B];
+#pragma unroll
+        for (int i = 0; i < B; i++) buf[i] = pp[c0 * ROW + min(tid + 256 * i, n * ROW - 1)]; // clamped: not stored
+        __syncthreads(); // the chunks before are consumed
+#pragma unroll
+        for (int i = 0; i < B; i++)
+            if (tid + 256 * i < n * ROW) part[tid + 256 * i] = buf[i];
+        __syncthreads();
+        if (tid < 64) {
+            const float m = tid < n ? part[tid * ROW].x : -INFINITY;
+            float mx = m;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const float up = __shfl_up(mx, o, 64);
+                if (tid >= o) mx = fmaxf(mx, up);
+            }
+            mx = fmaxf(mx, M);
+            float prev = __shfl_up(mx, 1, 64);
+            if (tid == 0) prev = M;
+            if (tid < n) {
+                fo[tid] = __expf(prev - mx);
+                fc[tid] = __expf(m - mx);
+            }
+            M = __shfl(mx, n - 1, 64);
+        }
+        __syncthreads();
+        if (tid < 128) {
+            const float *pf = (const float *)part;
+#pragma unroll 8
+            for (int c = 0; c < n; c++) {
+                L = fmaf(pf[c * 2 * ROW + 1], fc[c], L * fo[c]);
+                v = fmaf(pf[c * 2 * ROW + 2 + tid], fc[c], v * fo[c]);
+            }
+        }
+    }
+    if (tid < 128) {
+        const float inv = 1.0f / L;
+        out[h * 128 + tid] = v * inv;
+    }
+}
+
+hipError_t launch_attn_combine_one(const DecodeChunks &d, int n_heads, float *out, hipStream_t s)
+{
+    if (n_heads < 1 || d.max_chunks < 1 || !d.part || !out) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(attn_combine_one_kernel, dim3(n_heads), dim3(256), 0, s, d, out);
+    return hipGetLastError();
+}
+
 } // namespace jev

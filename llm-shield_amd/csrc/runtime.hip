@@ -469,7 +469,7 @@ int ensure_workspace(jev_ctx *c, int T, int n_out, int mode, int max_chunks, boo
     // its own input's
     HIP_TRY(c->xsum.ensure((size_t)std::max(T, n_out) * wide / 32 + (T <= 16 ? (size_t)T * f.ffn / 32 : 0) + 1));
     if (T == 1) {
-        HIP_TRY(c->x32.ensure((size_t)std::max<size_t>(f.hidden, 1)));
+        HIP_TRY(c->x32.ensure((size_t)std::max({f.hidden, c->qdim(), 1})));
         HIP_TRY(c->f32.ensure((size_t)2 * f.ffn));
         HIP_TRY(c->part.ensure((size_t)f.n_heads * std::max(1, max_chunks) * 130));
     } else {
@@ -1010,8 +1010,10 @@ int enqueue_forward(jev_ctx *c, const Plan &p, int mode, int n_rows, float *dout
         }
         {
             const QWeight *wo[1] = {&L.o};
-            int rc = linear(c, T, wo, 1, c->xt.p, c->xsum.p, nullptr, c->yo.p, D, s_o, 0,
-                            T == 1 ? &dchunks : nullptr);
+            const bool combined = T == 1 && dchunks.max_chunks > kCombineChunks;
+            if (combined) HIP_TRY(launch_attn_combine_one(dchunks, f.n_heads, c->x32.p, s));
+            int rc = linear(c, T, wo, 1, c->xt.p, c->xsum.p, combined ? c->x32.p : nullptr, c->yo.p, D, s_o, 0,
+                            T == 1 && !combined ? &dchunks : nullptr);
             if (rc) return rc;
         }
         CAP_TRY(cap_partials(c, cap, layer_tap(l, "attn_out"), c->yo.p, stored_parts(T, L.o, s_o), T, D));
