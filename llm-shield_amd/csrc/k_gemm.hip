@@ -986,7 +986,9 @@ static hipError_t launch_mode(const GemmArgs &a, hipStream_t s)
     // busiest CU does, so their time is whole workgroups per CU times a
     // workgroup's; four waves of 64 x 64, two workgroups at a time, run on
     // through a partial round, and past four rounds, where the power limit sets
-    // the clock, are the cheapest per row.  Relative times per workgroup from
+    // the clock, are the cheapest per row (in the model, 96-row stores of Q8_0
+    // took 2 % less at 2400 rows, 1 % more at 2812 and 3000; 64-row eight-wave
+    // SwiGLU 3 % more at 2400).  Relative times per workgroup from
     // launches of 520 to 3000 rows (us, 64 rows / 80 / 96 / the four waves): Q8_0
     // O, 700 rows 49.3 / 42.4 / 46.6 / 48.5, 900 52.4 / 62.3 / 50.4 / 52.1, 1500 82.2 /
     // 83.5 / 77.6 / 82.1; SwiGLU, 520 rows 141 / 125 / 135 / 141, 900 238 / 237 / 213 /
@@ -1006,7 +1008,7 @@ static hipError_t launch_mode(const GemmArgs &a, hipStream_t s)
             tall = 6;
         }
         const double share = (double)wgs(4, 4, 4) / kCUs, r4 = rounds(4);
-        const double four = (share == r4 ? r4 : share + 0.85) * (share > 4 ? 0.95 : 0.98);
+        const double four = (share == r4 ? r4 : share + 0.85) * (share <= 4 ? 0.98 : MODE == kGemmStore ? 0.90 : 0.95);
         if (one_seg && (four < best || (tall == 4 && share > 4)) && (MODE == kGemmSwiGlu || r4 > 2))
             return launch_bd<TYPE, MODE, 4, 4, 1, 2>(a, s);
         if (tall == 6) return launch_bd<TYPE, MODE, 6, 2, 1, 4, false, 8>(a, s);
