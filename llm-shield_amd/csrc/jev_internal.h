@@ -288,6 +288,15 @@ struct AttnSchedule {
     int run_blocks = 0; // 0: one workgroup walks all blocks of its tile
     int n_parts = 1;
     size_t floats = 0;  // workspace of the partials
+    int whole_ds = 1;   // ds of the best schedule without them
+    AttnSchedule whole() const
+    {
+        AttnSchedule s = *this;
+        s.ds = whole_ds;
+        s.run_blocks = 0;
+        s.floats = 0;
+        return s;
+    }
 };
 AttnSchedule attn_schedule(int n_tiles, int n_heads, int group, int max_blocks, double total_blocks);
 struct AttnArgs {

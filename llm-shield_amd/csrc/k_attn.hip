@@ -628,7 +628,7 @@ AttnSchedule attn_schedule(int n_tiles, int n_heads, int group, int max_blocks, 
     AttnSchedule best;
     best.n_parts = (max_blocks + kAttnPartBlocks - 1) / kAttnPartBlocks;
     const size_t floats = (size_t)n_tiles * n_heads * best.n_parts * kAttnPartFloats;
-    double best_us = 1e30;
+    double best_us = 1e30, whole_us = 1e30;
     // jobs of at most `longest` blocks, `avg` blocks per compute unit in all:
     // a second round starts when the work does not fit the first
     auto blocks = [](double jobs, double longest, double avg) {
@@ -639,6 +639,10 @@ AttnSchedule attn_schedule(int n_tiles, int n_heads, int group, int max_blocks, 
         const double avg = total_blocks * wide * ds / kCUs;
         double jobs = n_tiles * wide * ds;
         double us = blocks(jobs, max_blocks, avg) * kBlock[i] + kStart * std::ceil(jobs / kCUs);
+        if (us < whole_us) {
+            whole_us = us;
+            best.whole_ds = ds;
+        }
         if (us < best_us) {
             best_us = us;
             best.ds = ds;

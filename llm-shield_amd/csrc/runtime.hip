@@ -71,6 +71,7 @@ struct DevBuf {
         }
         hipError_t e = hipMalloc((void **)&p, std::max<size_t>(need, 1) * sizeof(T));
         if (e == hipSuccess) n = need;
+        else (void)hipGetLastError(); // returned here: the next launch's check must not find it
         return e;
     }
     void release()
@@ -352,6 +353,24 @@ int upload_vector(int type, int64_t count, const void *bytes, float **dst)
     return JEV_OK;
 }
 
+// The split attention's partials (apart) only make a pass faster.  Where another
+// allocation of the context finds no room (e), they are given back and it is
+// tried once more; the next split pass allocates them anew, or runs whole.
+bool give_back_partials(jev_ctx *c, hipError_t e)
+{
+    if (e != hipErrorOutOfMemory || !c->apart.p) return false;
+    if (hipDeviceSynchronize() != hipSuccess) return false; // queued work may still read them
+    c->apart.release();
+    return true;
+}
+
+template <typename T>
+hipError_t grow(jev_ctx *c, DevBuf<T> &b, size_t need)
+{
+    const hipError_t e = b.ensure(need);
+    return give_back_partials(c, e) ? b.ensure(need) : e;
+}
+
 // KvCache.EnsureCapacity (KvCache.cs:48-70): doubles until it fits and copies
 // the populated prefix of every head.
 int kv_ensure(jev_ctx *c, int required)
@@ -363,7 +382,14 @@ int kv_ensure(jev_ctx *c, int required)
     size_t bytes = heads * cap * c->cfg.head_dim * sizeof(float);
     void *buf[4] = {nullptr, nullptr, nullptr, nullptr};
     hipError_t e = hipSuccess;
-    for (int i = 0; i < 4 && e == hipSuccess; i++) e = hipMalloc(&buf[i], bytes);
+    do {
+        for (void *&b : buf) {
+            if (b) continue; // a second round keeps what the first one got
+            e = hipMalloc(&b, bytes);
+            if (e != hipSuccess) break;
+        }
+        if (e != hipSuccess) (void)hipGetLastError();
+    } while (e != hipSuccess && give_back_partials(c, e));
     if (e != hipSuccess) {
         for (void *b : buf)
             if (b) (void)hipFree(b);
@@ -459,34 +485,34 @@ int ensure_workspace(jev_ctx *c, int T, int n_out, int mode, int max_chunks, boo
     const jev_config &f = c->cfg;
     size_t qkv = (size_t)c->qdim() + 2 * c->kvdim();
     size_t wide = std::max<size_t>({(size_t)f.hidden, (size_t)c->qdim(), (size_t)f.ffn});
-    HIP_TRY(c->h.ensure((size_t)T * f.hidden));
-    HIP_TRY(c->y.ensure((size_t)T * qkv * c->split_qkv(T)));
-    HIP_TRY(c->yo.ensure((size_t)T * f.hidden * c->split_o(T)));
-    HIP_TRY(c->ydown.ensure((size_t)T * f.hidden * c->split_down(T)));
-    HIP_TRY(c->q.ensure((size_t)T * c->qdim()));
+    HIP_TRY(grow(c, c->h, (size_t)T * f.hidden));
+    HIP_TRY(grow(c, c->y, (size_t)T * qkv * c->split_qkv(T)));
+    HIP_TRY(grow(c, c->yo, (size_t)T * f.hidden * c->split_o(T)));
+    HIP_TRY(grow(c, c->ydown, (size_t)T * f.hidden * c->split_down(T)));
+    HIP_TRY(grow(c, c->q, (size_t)T * c->qdim()));
     // [0, T * wide / 32): the block sums a GEMM reads; past it, the SwiGLU
     // output's, written by the small-batch SwiGLU GEMM while it still reads
     // its own input's
-    HIP_TRY(c->xsum.ensure((size_t)std::max(T, n_out) * wide / 32 + (T <= 16 ? (size_t)T * f.ffn / 32 : 0) + 1));
+    HIP_TRY(grow(c, c->xsum, (size_t)std::max(T, n_out) * wide / 32 + (T <= 16 ? (size_t)T * f.ffn / 32 : 0) + 1));
     if (T == 1) {
-        HIP_TRY(c->x32.ensure((size_t)std::max({f.hidden, c->qdim(), 1})));
-        HIP_TRY(c->f32.ensure((size_t)2 * f.ffn));
-        HIP_TRY(c->part.ensure((size_t)f.n_heads * std::max(1, max_chunks) * 130));
+        HIP_TRY(grow(c, c->x32, (size_t)std::max({f.hidden, c->qdim(), 1})));
+        HIP_TRY(grow(c, c->f32, (size_t)2 * f.ffn));
+        HIP_TRY(grow(c, c->part, (size_t)f.n_heads * std::max(1, max_chunks) * 130));
     } else {
         if (single_rows)
-            HIP_TRY(c->part.ensure((size_t)single_rows_group(T, max_chunks) * f.n_heads * std::max(1, max_chunks) * 130));
+            HIP_TRY(grow(c, c->part, (size_t)single_rows_group(T, max_chunks) * f.n_heads * std::max(1, max_chunks) * 130));
         size_t T16 = ((size_t)T + 15) & ~(size_t)15;
-        HIP_TRY(c->xt.ensure(T16 * std::max(f.hidden, c->qdim()) * 2));
-        HIP_TRY(c->ft.ensure(T16 * f.ffn * 2));
+        HIP_TRY(grow(c, c->xt, T16 * std::max(f.hidden, c->qdim()) * 2));
+        HIP_TRY(grow(c, c->ft, T16 * f.ffn * 2));
     }
     size_t nx = std::max(1, n_out);
-    HIP_TRY(c->xn.ensure(nx * f.hidden));
+    HIP_TRY(grow(c, c->xn, nx * f.hidden));
     if (mode == JEV_OUT_FULL || mode == JEV_OUT_LAST_FULL) {
-        HIP_TRY(c->logits.ensure(nx * (size_t)f.vocab));
-        if (nx >= 2) HIP_TRY(c->xt.ensure(std::max(c->xt.n, ((nx + 15) & ~(size_t)15) * f.hidden * 2)));
+        HIP_TRY(grow(c, c->logits, nx * (size_t)f.vocab));
+        if (nx >= 2) HIP_TRY(grow(c, c->xt, std::max(c->xt.n, ((nx + 15) & ~(size_t)15) * f.hidden * 2)));
     }
-    HIP_TRY(c->amax_v.ensure(std::max<size_t>(512, nx))); // argmax candidates: 512, or one per output row
-    HIP_TRY(c->amax_i.ensure(std::max<size_t>(512, nx)));
+    HIP_TRY(grow(c, c->amax_v, std::max<size_t>(512, nx))); // argmax candidates: 512, or one per output row
+    HIP_TRY(grow(c, c->amax_i, std::max<size_t>(512, nx)));
     return JEV_OK;
 }
 
@@ -625,8 +651,8 @@ int build_plan(jev_ctx *c, const int32_t *tokens, bool tokens_on_device, int T, 
         p.rows_independent = ok;
     }
 
-    HIP_TRY(c->ints.ensure(H.size() + 1));
-    HIP_TRY(c->tiles.ensure(tiles.size() + 1));
+    HIP_TRY(grow(c, c->ints, H.size() + 1));
+    HIP_TRY(grow(c, c->tiles, tiles.size() + 1));
     // Stage through pinned memory; wait until the previous upload has read it.
     HIP_TRY(hipEventSynchronize(c->copied));
     if (c->pin_ints_n < H.size() + 1) {
@@ -804,6 +830,16 @@ int enqueue_forward(jev_ctx *c, const Plan &p, int mode, int n_rows, float *dout
     const bool q51 = c->layers[0].q.type == kQ5_1; // per-weight below
     (void)q51;
     hipStream_t s = c->stream;
+
+    // The partials of a split attention, after everything else the call
+    // allocates (never under capture: decode steps have none).  Without room
+    // for them each tile runs whole, which takes no scratch and gives the same bits.
+    AttnSchedule attn = p.attn;
+    if (attn.floats > 0) {
+        const hipError_t e = c->apart.ensure(attn.floats);
+        if (e == hipErrorOutOfMemory) attn = attn.whole();
+        else HIP_TRY(e);
+    }
 
     const int s_o = c->split_o(T), s_down = c->split_down(T);
     const size_t stride_d = (size_t)T * D; // floats between partials of yo / ydown
@@ -996,7 +1032,7 @@ int enqueue_forward(jev_ctx *c, const Plan &p, int mode, int n_rows, float *dout
             aa.cap = c->cap;
             aa.scale = scale;
             aa.ot = c->xt.p;
-            aa.sched = p.attn;
+            aa.sched = attn;
             aa.part = c->apart.p;
             {
                 ProfScope ps(c, JEV_PROF_ATTN, 4.0 * f.head_dim * f.n_heads * p.visible_pairs,
@@ -1228,7 +1264,6 @@ int prepare(jev_ctx *c, const int32_t *tokens, bool on_device, int T, const jev_
     if (rc) return rc;
     rc = build_plan(c, tokens, on_device, T, layout, mode, rows, n_rows, p);
     if (rc) return rc;
-    HIP_TRY(c->apart.ensure(p.attn.floats));
     return ensure_workspace(c, T, p.n_out, mode, p.max_chunks, p.single_rows);
 }
 
@@ -1539,7 +1574,13 @@ int jev_kv_snapshot_device(jev_ctx *c, int32_t length, jev_snapshot **out)
     sn->head_dim = f.head_dim;
     sn->length = length;
     sn->floats = 2 * (size_t)f.n_layers * f.n_kv_heads * length * f.head_dim;
-    hipError_t e = hipMalloc((void **)&sn->data, std::max<size_t>(sn->floats, 1) * sizeof(float));
+    auto alloc = [&] {
+        hipError_t r = hipMalloc((void **)&sn->data, std::max<size_t>(sn->floats, 1) * sizeof(float));
+        if (r != hipSuccess) (void)hipGetLastError();
+        return r;
+    };
+    hipError_t e = alloc();
+    if (give_back_partials(c, e)) e = alloc();
     if (e != hipSuccess) {
         const size_t bytes = sn->floats * sizeof(float);
         delete sn;
@@ -1608,7 +1649,7 @@ int jev_forward(jev_ctx *c, const int32_t *tokens, int32_t T, const jev_layout *
     if (need && (!out || out_len < need)) return fail(JEV_EINVAL, "Expected room for %zu outputs, got %zu.", need, out_len);
     float *dout = nullptr;
     if (need) {
-        HIP_TRY(c->logits.ensure(std::max(c->logits.n, need)));
+        HIP_TRY(grow(c, c->logits, std::max(c->logits.n, need)));
         dout = c->logits.p;
     }
     rc = enqueue_forward(c, p, mode, n_rows, dout, nullptr, &call, true);
@@ -1637,8 +1678,8 @@ int jev_capture(jev_ctx *c, const int32_t *tokens, int32_t T, jev_sink sink, voi
     Plan p;
     rc = prepare(c, tokens, false, T, nullptr, JEV_OUT_LAST_FULL, nullptr, 0, p);
     if (rc) return rc;
-    HIP_TRY(c->cap32.ensure((size_t)T * std::max(c->cfg.hidden, c->qdim())));
-    HIP_TRY(c->logits.ensure(std::max(c->logits.n, (size_t)c->cfg.vocab)));
+    HIP_TRY(grow(c, c->cap32, (size_t)T * std::max(c->cfg.hidden, c->qdim())));
+    HIP_TRY(grow(c, c->logits, std::max(c->logits.n, (size_t)c->cfg.vocab)));
     Capture cap;
     rc = enqueue_forward(c, p, JEV_OUT_LAST_FULL, 0, c->logits.p, nullptr, &call, false, &cap);
     if (rc) {
@@ -1733,7 +1774,7 @@ int jev_decode_greedy(jev_ctx *c, int32_t first, int32_t n_steps, int32_t *token
     const int start = c->len, end = start + n_steps;
     rc = kv_ensure(c, end);
     if (rc) return rc;
-    HIP_TRY(c->dec_state.ensure((size_t)n_steps + 3));
+    HIP_TRY(grow(c, c->dec_state, (size_t)n_steps + 3));
     int32_t *state = c->dec_state.p, *out = c->dec_state.p + 3;
     const int32_t init[3] = {start, 0, first};
     HIP_TRY(hipMemcpy(state, init, sizeof(init), hipMemcpyHostToDevice));
@@ -1742,7 +1783,7 @@ int jev_decode_greedy(jev_ctx *c, int32_t first, int32_t n_steps, int32_t *token
     if (rc) return rc;
     p.max_chunks = (end + kDecodeKeys - 1) / kDecodeKeys; // grid for the longest step; shorter ones exit early
     rc = ensure_workspace(c, 1, p.n_out, JEV_OUT_LAST_FULL, p.max_chunks);
-    if (!rc && c->logits.ensure(std::max(c->logits.n, (size_t)c->cfg.vocab)) != hipSuccess) rc = fail(JEV_ENOMEM, "logits");
+    if (!rc && grow(c, c->logits, std::max(c->logits.n, (size_t)c->cfg.vocab)) != hipSuccess) rc = fail(JEV_ENOMEM, "logits");
     if (rc) return rc;
     auto step = [&]() -> int {
         int r = enqueue_forward(c, p, JEV_OUT_LAST_FULL, 0, c->logits.p, state);
@@ -1870,8 +1911,8 @@ int jev_decode_rows_greedy(jev_ctx *c, int32_t shared, int32_t n_rows, const int
     p.max_chunks = (max_limit + kDecodeKeys - 1) / kDecodeKeys; // grid for the longest step
     rc = ensure_workspace(c, n_rows, p.n_out, JEV_OUT_FULL, p.max_chunks, p.single_rows);
     if (rc) return rc;
-    HIP_TRY(c->logits.ensure(std::max(c->logits.n, (size_t)n_rows * c->cfg.vocab)));
-    HIP_TRY(c->dec_state.ensure((size_t)n_rows * (n_steps + 1)));
+    HIP_TRY(grow(c, c->logits, std::max(c->logits.n, (size_t)n_rows * c->cfg.vocab)));
+    HIP_TRY(grow(c, c->dec_state, (size_t)n_rows * (n_steps + 1)));
     int32_t *rowstep = c->dec_state.p, *out = c->dec_state.p + n_rows;
     HIP_TRY(hipMemsetAsync(rowstep, 0, (size_t)n_rows * sizeof(int32_t), c->stream));
     // two or more rows: every row is its own attention tile (the rows' slots
