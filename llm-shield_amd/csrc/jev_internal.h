@@ -311,6 +311,7 @@ struct AttnArgs {
     float scale = 0.f;
     uint16_t *ot = nullptr; // context pair, operand-tile layout, K = qdim
     hipEvent_t ev_start = nullptr, ev_stop = nullptr; // optional dispatch-stamped timing
+    hipEvent_t ev_merge_start = nullptr, ev_merge_stop = nullptr; // of a split pass's merge
 };
 hipError_t launch_attn_tree(const AttnArgs &a, hipStream_t s);
 
@@ -367,7 +368,8 @@ hipError_t launch_attn_combine(const AttnCombineArgs &a, hipStream_t s);
 // what one workgroup per head here reads once (Q8_0 O in the model, us, inside ->
 // ahead: 93 chunks 24.4 -> 11.6, 63 18.3 -> 9.9, 24 10.3 -> 8.9; 9, Q5_1, 8.1 -> 8.2).
 constexpr int kCombineChunks = 16;
-hipError_t launch_attn_combine_one(const DecodeChunks &d, int n_heads, float *out, hipStream_t s);
+hipError_t launch_attn_combine_one(const DecodeChunks &d, int n_heads, float *out, hipEvent_t ev_start, hipEvent_t ev_stop,
+                                   hipStream_t s);
 
 // Verdict-row head: for each output b, logits[b][i] = dot(norm(h[outputs[b]]), W[rows[i]]).
 struct HeadRowsArgs {

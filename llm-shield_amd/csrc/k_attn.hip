@@ -687,7 +687,7 @@ hipError_t launch_attn_tree(const AttnArgs &args, hipStream_t s)
     };
     if (c.run_blocks > 0) {
         launch_ds(std::integral_constant<int, kSplit>{});
-        hipLaunchKernelGGL(attn_merge_kernel, dim3(a.n_heads, a.n_tiles), dim3(256), 0, s, a);
+        launch_stamped(a.ev_merge_start, a.ev_merge_stop, attn_merge_kernel, dim3(a.n_heads, a.n_tiles), dim3(256), 0, s, a);
     } else if (c.n_parts > 1) {
         launch_ds(std::integral_constant<int, kMerged>{});
     } else {
@@ -1152,10 +1152,11 @@ __global__ __launch_bounds__(256) void attn_combine_one_kernel(DecodeChunks d, f
     }
 }
 
-hipError_t launch_attn_combine_one(const DecodeChunks &d, int n_heads, float *out, hipStream_t s)
+hipError_t launch_attn_combine_one(const DecodeChunks &d, int n_heads, float *out, hipEvent_t ev_start, hipEvent_t ev_stop,
+                                   hipStream_t s)
 {
     if (n_heads < 1 || d.max_chunks < 1 || !d.part || !out) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(attn_combine_one_kernel, dim3(n_heads), dim3(256), 0, s, d, out);
+    launch_stamped(ev_start, ev_stop, attn_combine_one_kernel, dim3(n_heads), dim3(256), 0, s, d, out);
     return hipGetLastError();
 }
 

@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <thread>
 #include <vector>
@@ -1016,6 +1017,9 @@ int enqueue_forward(jev_ctx *c, const Plan &p, int mode, int n_rows, float *dout
                     da.ev_stop = ps.z;
                     HIP_TRY(launch_attn_decode(da, s));
                 }
+                ProfScope pc(c, JEV_PROF_DECODE_ATTN, 0.0, 0.0, true);
+                ca.ev_start = pc.a;
+                ca.ev_stop = pc.z;
                 HIP_TRY(launch_attn_combine(ca, s));
             }
             CAP_TRY(cap_pair(c, cap, layer_tap(l, "attn_weighted"), c->xt.p, T, qdim));
@@ -1039,6 +1043,13 @@ int enqueue_forward(jev_ctx *c, const Plan &p, int mode, int n_rows, float *dout
                              8.0 * f.head_dim * f.n_kv_heads * p.kv_rows + 8.0 * T * qdim, true);
                 aa.ev_start = ps.a;
                 aa.ev_stop = ps.z;
+                // a split pass's merge: a launch of its own in the same class
+                std::optional<ProfScope> pm;
+                if (attn.run_blocks > 0) {
+                    pm.emplace(c, JEV_PROF_ATTN, 0.0, 0.0, true);
+                    aa.ev_merge_start = pm->a;
+                    aa.ev_merge_stop = pm->z;
+                }
                 HIP_TRY(launch_attn_tree(aa, s));
             }
             CAP_TRY(cap_pair(c, cap, layer_tap(l, "attn_weighted"), c->xt.p, T, qdim));
@@ -1047,7 +1058,10 @@ int enqueue_forward(jev_ctx *c, const Plan &p, int mode, int n_rows, float *dout
         {
             const QWeight *wo[1] = {&L.o};
             const bool combined = T == 1 && dchunks.max_chunks > kCombineChunks;
-            if (combined) HIP_TRY(launch_attn_combine_one(dchunks, f.n_heads, c->x32.p, s));
+            if (combined) {
+                ProfScope pc(c, JEV_PROF_DECODE_ATTN, 0.0, 0.0, true);
+                HIP_TRY(launch_attn_combine_one(dchunks, f.n_heads, c->x32.p, pc.a, pc.z, s));
+            }
             int rc = linear(c, T, wo, 1, c->xt.p, c->xsum.p, combined ? c->x32.p : nullptr, c->yo.p, D, s_o, 0,
                             T == 1 && !combined ? &dchunks : nullptr);
             if (rc) return rc;
