@@ -14,6 +14,28 @@ VOCAB = 2048
 ROWS = [5, 77, 1999]
 
 
+# 32 / 8 heads: tokens in all, of them new, workgroups that share a tile's output dims,
+# partitions to a run
+RUNS = [(2049, 200, 2, 1), (2700, 200, 1, 1), (4396, 30, 4, 1), (4396, 300, 1, 2), (12450, 250, 1, 4), (12200, 600, 1, 8)]
+
+
+@pytest.mark.parametrize("total,new,ds,parts", RUNS)
+def test_runs_of_several_partitions_give_the_whole_prompt_s_bits(gpu, total, new, ds, parts):
+    # a workgroup whose run holds several partitions stores each one's partial as
+    # it goes on to the next; the whole prompt merges them in its registers
+    cfg = jev.ModelConfig(n_layers=1, hidden=256, n_heads=32, n_kv_heads=8, head_dim=128, ffn=512, vocab=VOCAB,
+                          initial_kv_capacity=64)
+    model = jev.SynthModel(cfg, jev.TYPE_Q8_0).open(0)
+    tokens = jev.random_tokens(total, VOCAB, 22)
+    outputs = [0, 1, new // 2, new - 2, new - 1]
+    lay = jev.TokenLayout.tree(0, total, [], total).with_outputs([total - new + o for o in outputs])
+    whole = model.forward_layout(tokens, lay, jev.OUT_FULL)
+    model.kv_truncate(total - new)
+    lay = jev.TokenLayout.tree(total - new, new, [], new).with_outputs(outputs)
+    assert np.array_equal(whole, model.forward_layout(tokens[total - new:], lay, jev.OUT_FULL))
+    model.close()
+
+
 @pytest.mark.parametrize("heads,kv", [(4, 2), (6, 1), (32, 8)])
 def test_suffix_bits_do_not_depend_on_the_split(gpu, heads, kv):
     # prompts whose last token sits around the partition edges: the same tokens as a

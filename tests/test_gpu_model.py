@@ -128,14 +128,18 @@ def test_tree_equals_branches_alone_bitwise_other_types(gpu, t):
         assert np.array_equal(alone[b], tree[b]), b
 
 
-@pytest.mark.parametrize("trunk", [2100, 4100])
+# trunk: (workgroups that share a tile's 128 output dims, partitions, grid z) of the tree pass
+TREE_FORMS = {900: (4, "one", 4), 1100: (2, "merged", 2), 1500: (2, "split", 4), 2100: (1, "split", 3),
+              4100: (1, "split", 5), 6000: (1, "merged", 1), 12000: (1, "split", 6)}
+
+
+@pytest.mark.parametrize("trunk", TREE_FORMS)
 def test_tree_equals_branches_alone_across_attention_grids(model, trunk):
-    # The attention grid has one workgroup per 32-token tile and KV head; grids
-    # smaller than the GPU split the 128 output dims over 2 (up to 255
-    # workgroups) or 4 (up to 64) workgroups.  With this model's 2 KV heads a
-    # 4100-token tree pass computes all dims per workgroup, a 2100-token one
-    # splits them in two, the short branches alone in four.  The bits must not
-    # change.
+    # A pass's attention is cut by its tiles and contexts: 1, 2 or 4 workgroups
+    # share a tile's output dims, and the 1024-key partitions are one, merged
+    # inside the workgroup or in runs of their own (at 12000 two partitions to a
+    # run).  The branches alone over 1500 keys and more take runs of one
+    # partition.  The bits must not change.
     prefix = jev.random_tokens(trunk, 2048, 21)
     branches = [jev.random_tokens(n, 2048, 90 + n) for n in (40, 3)]
     m = fresh(model)
@@ -280,8 +284,9 @@ def test_other_block_types(gpu, t):
 @pytest.mark.parametrize("n", [70, 600])
 def test_projection_segments_off_the_wide_tile_grid(gpu, t, n):
     # 3 query heads over 1 KV head: the fused QKV segments (384, 128, 128 rows)
-    # do not split on 256-row boundaries, so the projections take the
-    # dequant-in-LDS GEMM (small and large batch shapes) instead of B-direct.
+    # do not split on 256-row boundaries: four-wave tiles of 64 columns at 70
+    # rows, and at 600 eight-wave tiles of 256, where each wave finds the
+    # segment of its own columns.
     cfg = tiny_config(n_heads=3, n_kv_heads=1, initial_kv_capacity=1024)
     synth = jev.SynthModel(cfg, t)
     m = synth.open(0)
