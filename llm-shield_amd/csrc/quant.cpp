@@ -118,6 +118,9 @@ QLayout qlayout(int type, int64_t rows, int64_t cols)
 
 static void parallel_rows(int64_t rows, int threads, const std::function<void(int64_t, int64_t)> &fn);
 
+// Bit i of a 4-bit value to bit 4 of byte i.
+static inline uint32_t fifth_bits(uint32_t x) { return ((x * 0x00204081u) & 0x01010101u) << 4; }
+
 // GGUF blocks -> tiles.  Element (r, k) of a block pair goes to lane
 // l = 16 (k % 32 / 8) + r % 16; see the layout description in jev_internal.h.
 bool repack_host(int type, int64_t rows, int64_t cols, const void *gguf, void *dst, int threads)
@@ -173,17 +176,25 @@ bool repack_host(int type, int64_t rows, int64_t cols, const void *gguf, void *d
                         for (int i = 0; i < 4; i++) dq[i] = (uint8_t)(nib(8 * g + i) | (nib(8 * g + i + 4) << 4));
                         continue;
                     }
-                    uint32_t q[8], word = 0;
-                    for (int i = 0; i < 8; i++) q[i] = nib(8 * g + i) | (((qh >> (8 * g + i)) & 1u) << 4);
-                    for (int i = 0; i < 6; i++) word |= q[i] << (5 * (i / 2) + 16 * (i % 2));
-                    word |= (q[6] >> 4) << 15 | (q[7] >> 4) << 31;
+                    // the eight quants as bytes, elements 8 g .. + 3 in a and + 4 .. + 7 in b, then
+                    // each field's bits moved as they lie (element by element, binding 3072 x 9216 took
+                    // about 90 ms of eight host threads instead of 67)
+                    uint32_t a, b;
+                    std::memcpy(&a, qs + 8 * (g & 1), 4);
+                    std::memcpy(&b, qs + 8 * (g & 1) + 4, 4);
+                    const uint32_t high = (qh >> (8 * g)) & 0xffu;
+                    a = ((g < 2 ? a : a >> 4) & 0x0f0f0f0fu) | fifth_bits(high & 15u);
+                    b = ((g < 2 ? b : b >> 4) & 0x0f0f0f0fu) | fifth_bits(high >> 4);
+                    const uint32_t word = (a & 0x1fu) | (a & 0x1f00u) << 8 | ((a >> 11) & 0x3e0u) | ((a >> 3) & 0x3e00000u) |
+                                          (b & 0x1fu) << 10 | (b & 0x1f00u) << 18 | ((b >> 5) & 0x8000u) | ((b & 0x10000000u) << 3);
                     std::memcpy(dq, &word, 4);
                     uint8_t *lo = out + L.qh + tile * 128 + 2 * lane;
-                    lo[0] |= (uint8_t)((q[6] & 15u) << (4 * bb));
-                    lo[1] |= (uint8_t)((q[7] & 15u) << (4 * bb));
+                    lo[0] |= (uint8_t)(((b >> 16) & 15u) << (4 * bb));
+                    lo[1] |= (uint8_t)(((b >> 24) & 15u) << (4 * bb));
                     // the byte copy: element 8 g + i at byte 8 bb + i of lane 16 g + r
                     uint8_t *db = out + L.qb + tile * 1024 + 16 * lane + 8 * bb;
-                    for (int i = 0; i < 8; i++) db[i] = (uint8_t)q[i];
+                    std::memcpy(db, &a, 4);
+                    std::memcpy(db + 4, &b, 4);
                 }
             }
         }
