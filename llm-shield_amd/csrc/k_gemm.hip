@@ -39,6 +39,7 @@
 // neighbouring tiles on one XCD share weight and activation tiles in its L2.
 #include "jev_dev.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace jev {
@@ -125,6 +126,10 @@ __device__ __forceinline__ half8_t decode_b_frag(const BChunk &c, int bb)
 //   4 x 2 and 4 x 4 tiles: two pairs; 4 x 2 with plain FMAs but for Q4_0 (Q5_1
 //     QKV 1500 rows 160 -> 149, down 236 -> 219, SwiGLU 640 193 -> 178; SwiGLU
 //     256 rows Q8_0 81 -> 72, Q5_1 100 -> 84)
+//   5 x 2 and 6 x 2 of Q4_0 and Q5_1: one pair.  With two they need 4 to 14
+//     registers past the 128 of two workgroups per CU, and the scratch they took
+//     cost more than the lag gives (Q5_1 SwiGLU 520 rows 165 -> 145 us; Q4_0 calls
+//     of 768 rows: down 106 -> 97, QKV 75 -> 68)
 //   2 x 1: two pairs and plain FMAs (Q8_0 QKV 96 rows 14.9 -> 13.9, Q4_0 down
 //     20.6 -> 18.6)
 //   1 x 1, 1 x 2: one pair (Q8_0 down 32 rows 12.6 -> 11.8, Q5_1 16.3 -> 15.0)
@@ -133,6 +138,7 @@ __device__ __forceinline__ half8_t decode_b_frag(const BChunk &c, int bb)
 //     room in its 128 registers (SwiGLU 200 rows 97 -> 68)
 constexpr int bd_lag(int type, int tm, int tn, int nw)
 {
+    if (tm >= 5 && type != kQ8_0) return 1;
     return tm * tn >= 8 || (tm == 2 && tn == 1) || (type == kQ5_1 && nw >= 14) ? 2 : tm == 1 ? 1 : 0;
 }
 constexpr bool bd_plain_scale(int type, int tm, int tn, int nw)
@@ -984,17 +990,22 @@ static hipError_t launch_mode(const GemmArgs &a, hipStream_t s)
     // The height of the tile by the rounds its grid takes.  Eight waves of 64,
     // 80 or 96 rows x 32 columns (two such workgroups fit a CU) finish when the
     // busiest CU does, so their time is whole workgroups per CU times a
-    // workgroup's; four waves of 64 x 64, two workgroups at a time, run on
-    // through a partial round, and past four rounds, where the power limit sets
-    // the clock, are the cheapest per row (in the model, 96-row stores of Q8_0
-    // took 2 % less at 2400 rows, 1 % more at 2812 and 3000; 64-row eight-wave
-    // SwiGLU 3 % more at 2400).  Relative times per workgroup from
-    // launches of 520 to 3000 rows (us, 64 rows / 80 / 96 / the four waves): Q8_0
-    // O, 700 rows 49.3 / 42.4 / 46.6 / 48.5, 900 52.4 / 62.3 / 50.4 / 52.1, 1500 82.2 /
-    // 83.5 / 77.6 / 82.1; SwiGLU, 520 rows 141 / 125 / 135 / 141, 900 238 / 237 / 213 /
-    // 251.  Q5_1 has no registers for 96 rows, nor for its byte quants in the
-    // four-wave tile.
-    constexpr double k80 = TYPE == kQ8_0 ? 1.26 : TYPE == kQ4_0 ? 1.34 : MODE == kGemmStore ? 1.31 : 1.48, k96 = 1.42;
+    // workgroup's; four waves of 64 x 64, up to three workgroups at a time, run on
+    // through a partial round, and among many rounds, where the power limit sets
+    // the clock, are the cheapest per row.  The relative times per workgroup are
+    // of kernels between others (us, four waves / 64 rows / 80 / 96): Q8_0 O, 700
+    // rows 46.0 / 47.3 / 41.2 / 45.2, 900 49.6 / 50.0 / 59.8 / 48.8, 3000 139.9 /
+    // 144.1 / 149.8 / 145.5; Q4_0 O, 700 rows 45.5 / 46.0 / 39.0 / 42.6, 1500 77.0 /
+    // 76.2 / 75.3 / 73.6; SwiGLU, 520 rows of Q8_0 133 / 135 / 119 / 131, 900 of Q4_0
+    // 214 / 210 / 209 / 187; Q5_1 SwiGLU 700 rows 64 / 80: 212 / 202.  In a
+    // single matmul, between a pair split and a sum of partials, a store of 80 rows
+    // can be up to 5 % behind the four waves that it is ahead of in a prompt (Q4_0
+    // at 1150 rows: QKV 102 against 97, the prompt's four layers 2598 against 2687).
+    // Against four waves throughout, four 3B layers take, 700 / 900 / 1500 / 2400
+    // rows: Q4_0 1828 -> 1683, 2164 -> 1992, 3176 -> 3120, 5061 -> 5005; Q8_0 1839 ->
+    // 1738, 2173 -> 2114, 3228 -> 3212, 5169 -> 5124.  Q5_1 has no registers for 96
+    // rows, nor for its byte quants in the four-wave tile.
+    constexpr double k80 = MODE == kGemmStore ? 1.28 : 1.24, k96 = 1.41;
     auto rounds = [&](int tm) { return (double)((wgs(tm, 2, 8) + kCUs - 1) / kCUs); };
     double best = rounds(4);
     int tall = 4;
@@ -1007,8 +1018,9 @@ static hipError_t launch_mode(const GemmArgs &a, hipStream_t s)
             best = rounds(6) * k96;
             tall = 6;
         }
+        constexpr double k64 = TYPE == kQ4_0 ? 0.96 : MODE == kGemmStore ? 0.90 : 0.95; // four waves
         const double share = (double)wgs(4, 4, 4) / kCUs, r4 = rounds(4);
-        const double four = (share == r4 ? r4 : share + 0.85) * (share <= 4 ? 0.98 : MODE == kGemmStore ? 0.90 : 0.95);
+        const double four = std::min(r4, share + 0.88) * k64;
         if (one_seg && (four < best || (tall == 4 && share > 4)) && (MODE == kGemmSwiGlu || r4 > 2))
             return launch_bd<TYPE, MODE, 4, 4, 1, 2>(a, s);
         if (tall == 6) return launch_bd<TYPE, MODE, 6, 2, 1, 4, false, 8>(a, s);
@@ -1032,7 +1044,9 @@ hipError_t launch_gemm(const GemmArgs &a, hipStream_t s)
         return hipErrorInvalidValue; // every split non-empty; SwiGLU needs whole sums
     for (int i = 0; i < a.nseg; i++) {
         if (a.seg[i].type != a.seg[0].type || a.seg[i].cols != a.K) return hipErrorInvalidValue;
-        // every segment but the last must tile exactly (both tile widths divide 64)
+        // every segment but the last is whole four-wave tiles of 64 or 128 columns
+        // and whole wave shares of the wider workgroups (256-column four-wave
+        // tiles ask for more: one_seg, and the check of the fold below)
         if (a.mode == kGemmStore && i + 1 < a.nseg && a.seg[i].rows % 128 != 0) return hipErrorInvalidValue;
     }
     if (a.mode == kGemmSwiGlu && (a.nseg != 2 || a.seg[0].rows != a.seg[1].rows || a.seg[0].rows % 32 != 0))

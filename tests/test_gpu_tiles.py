@@ -50,7 +50,7 @@ def test_matmul_rows_do_not_depend_on_the_height_of_a_large_batch_tile(gpu, t):
     raw = jev.synth_tensor("tall", t, rows, cols)
     x = np.random.default_rng(6).standard_normal((1700, cols)).astype(np.float32)
     full = matmul_gpu(t, raw, rows, cols, x, 1700)
-    # 80-row tiles at 700, 96-row at 900 and 1500, 64-row between
+    # 80-row tiles at 700, 96-row ones at 1500 (Q5_1: 64-row), 64-row or four-wave ones between
     for n in (641, 700, 720, 721, 768, 900, 960, 961, 1100, 1500, 1536, 1537):
         lo = (n * 7) % (1700 - n)
         assert np.array_equal(full[lo:lo + n], matmul_gpu(t, raw, rows, cols, x[lo:lo + n], n)), n
