@@ -43,8 +43,9 @@ int64_t row_bytes(int type, int64_t cols);
 //                          Q8_0's order (lane l's 16 bytes at 16 l), for the
 //                          kernels of two or more tokens: one byte permute and
 //                          one packed subtraction per two weights instead of the
-//                          nibble and fifth-bit assembly (the one-token GEMV and the
-//                          few-row vocabulary head keep the 5-bit fields, whose
+//                          nibble and fifth-bit assembly; and for the Integer
+//                          strategy, whose operand they are (the one-token GEMV and
+//                          the few-row vocabulary head keep the 5-bit fields, whose
 //                          bytes they stream)
 constexpr int kTileRows = 16, kTileK = 64;
 struct QWeight {

@@ -146,11 +146,12 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_kernel(GemmI8Args a)
     const int rgw = blockIdx.x * 4 + wave;
     const int tile0 = __builtin_amdgcn_readfirstlane(min(rgw, RG - 1) * KP);
     const uint32_t tiles = (uint32_t)RG * KP;
-    constexpr bool BYTES = TYPE == kQ8_0;
-    const rsrc_t rq = make_rsrc(w.qs, tiles * (BYTES ? 1024u : 512u));
+    // Q5_1 from its byte copy, which is the operand as it lies: the kernel is short
+    // of vector issue, not of bytes (3072 x 9216, 1 / 256 rows: from the packed
+    // 5-bit fields 41.9 / 68.0 us a call, from the bytes 34.5 / 56.5)
+    constexpr bool BYTES = TYPE != kQ4_0;
+    const rsrc_t rq = make_rsrc(TYPE == kQ5_1 ? w.qb : w.qs, tiles * (BYTES ? 1024u : 512u));
     const rsrc_t rd = make_rsrc(w.d, tiles * (uint32_t)tile_d_bytes(TYPE));
-    rsrc_t rh;
-    if (TYPE == kQ5_1) rh = make_rsrc(w.qh, tiles * 128u);
     const rsrc_t rx = make_rsrc(a.xq, (uint32_t)a.T16 * nb * 32u);
     const rsrc_t rxd = make_rsrc(a.xd, (uint32_t)a.T16 * nb * 4u);
     rsrc_t raux;
@@ -209,9 +210,8 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_kernel(GemmI8Args a)
 
     // ---- weight slot of tile pair kp (clamped past the last)
     struct WStage {
-        uint4 q;     // Q8_0 16 bytes, nibbles 8 in .x, .y
-        uint32_t qh; // Q5_1: QWeight::qh's 16 bits of the lane
-        uint2 dm;    // two scales (.x; Q5_1: mins in .y)
+        uint4 q;  // bytes (Q8_0, Q5_1) 16, nibbles 8 in .x, .y
+        uint2 dm; // two scales (.x; Q5_1: mins in .y)
     };
     auto load_w = [&](WStage &s, int kp) __attribute__((always_inline)) {
         kp = min(kp, KP - 1);
@@ -223,7 +223,6 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_kernel(GemmI8Args a)
             s.q = make_uint4(v.x, v.y, 0u, 0u);
         }
         if (TYPE == kQ5_1) {
-            s.qh = __builtin_amdgcn_raw_buffer_load_b16(rh, 2 * lane, tile * 128, 0);
             s.dm = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rd, 8 * rl, tile * 128, 0));
         } else {
             s.dm.x = __builtin_amdgcn_raw_buffer_load_b32(rd, 4 * rl, tile * 64, 0);
@@ -242,26 +241,18 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_kernel(GemmI8Args a)
     auto compute = [&](const WStage &s, int kp, int buf, int lb0, auto check) __attribute__((always_inline)) {
         constexpr bool CHECK = decltype(check)::value;
         uint32_t wq[2][2]; // [block][dword]: the lane's 8 quants of each block
-        if (TYPE == kQ8_0) {
-            wq[0][0] = s.q.x ^ 0x80808080u;
-            wq[0][1] = s.q.y ^ 0x80808080u;
-            wq[1][0] = s.q.z ^ 0x80808080u;
-            wq[1][1] = s.q.w ^ 0x80808080u;
+        if (BYTES) {
+            constexpr uint32_t bias = TYPE == kQ8_0 ? 0x80808080u : 0u; // Q8_0's are stored as q + 128
+            wq[0][0] = s.q.x ^ bias;
+            wq[0][1] = s.q.y ^ bias;
+            wq[1][0] = s.q.z ^ bias;
+            wq[1][1] = s.q.w ^ bias;
         } else {
 #pragma unroll
             for (int bb = 0; bb < 2; bb++) {
                 const uint32_t v = bb ? s.q.y : s.q.x;
-                if (TYPE == kQ5_1) {
-                    // element pairs (QWeight's word: 0 | 1, 2 | 3, 4 | 5; 6 | 7 with qh)
-                    const uint32_t p0 = v & 0x001f001fu, p1 = (v >> 5) & 0x001f001fu, p2 = (v >> 10) & 0x001f001fu;
-                    const uint32_t lo = __builtin_amdgcn_perm(0u, s.qh, 0x0c010c00u) >> (4 * bb); // bytes 0 and 2
-                    const uint32_t p3 = (lo & 0x000f000fu) | ((v >> 11) & 0x00100010u);
-                    wq[bb][0] = __builtin_amdgcn_perm(p1, p0, 0x06040200u);
-                    wq[bb][1] = __builtin_amdgcn_perm(p3, p2, 0x06040200u);
-                } else {
-                    wq[bb][0] = v & 0x0f0f0f0fu;
-                    wq[bb][1] = (v >> 4) & 0x0f0f0f0fu;
-                }
+                wq[bb][0] = v & 0x0f0f0f0fu;
+                wq[bb][1] = (v >> 4) & 0x0f0f0f0fu;
             }
         }
 #pragma unroll
