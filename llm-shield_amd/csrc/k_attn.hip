@@ -44,7 +44,8 @@
 //
 // Decode kernel (attn_decode_kernel): one query per head, split over chunks
 // of 64 logical keys per KV head; the chunks are combined in ascending order
-// by the consumer, the O projection's GEMV, while it stages its input.
+// by the consumer, the O projection's GEMV, while it stages its input, past
+// kCombineChunks of them by attn_combine_one_kernel ahead of it.
 #include "jev_dev.h"
 
 #include <cmath>
@@ -702,7 +703,8 @@ hipError_t launch_attn_tree(const AttnArgs &args, hipStream_t s)
 // and V rows are staged in LDS once with coalesced loads and serve the
 // group's query heads (wave w takes heads w, w + 4, ...).  Scores: lane =
 // key, fp32 dot over 128 dims; weighted sum: lane = two dims.  Each chunk
-// leaves (max, sum, o[128]) per head.  The GEMV of the O projection merges
+// leaves (max, sum, o[128]) per head.  The GEMV of the O projection (of many
+// chunks attn_combine_one_kernel, of several tokens attn_combine_kernel) merges
 // the chunks in ascending order while staging its input (the kernel boundary
 // makes the partials visible; a last-to-finish merge here would need a
 // device-scope fence per workgroup, an L2 write-back and invalidate on this

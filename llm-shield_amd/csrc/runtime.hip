@@ -955,7 +955,7 @@ int enqueue_forward(jev_ctx *c, const Plan &p, int mode, int n_rows, float *dout
             da.part = c->part.p;
             da.rope_fused = cap ? 0 : 1;
             da.rope = ra;
-            // the O GEMV merges the chunks while staging its input
+            // the O GEMV merges the chunks while staging its input (many: a launch ahead of it does)
             dchunks.part = da.part;
             dchunks.max_chunks = da.max_chunks;
             dchunks.slot = da.slot;
